@@ -81,6 +81,10 @@ struct PlanError {
 // no GPU implementation exists.
 std::unique_ptr<Node> build_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why);
+// C2C on the tile kernels (tile_plan.cpp); null, with *why untouched, where
+// they do not apply
+std::unique_ptr<Node> build_columns_node(const Problem &p, std::string *why);
+std::unique_ptr<Node> build_tile_fourstep_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_real_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_r2r_node(const Problem &p, std::string *why);
 // Q0.15 / Q0.7 problems (p.fixed_bits != 0): power-of-two n only.
@@ -176,6 +180,7 @@ hipError_t dft_f64_gpu(std::vector<double> &v, int64_t M, int64_t count);
 // exp(sign*2*pi*i*num/den) with num reduced exactly mod den, long double
 // evaluation rounded once to double.
 void unit_root(int64_t num, int64_t den, double *re, double *im);
+void unit_root_l(int64_t num, int64_t den, long double *re, long double *im);
 
 // Last error text for the calling thread (plan creation diagnostics).
 void set_last_error(const std::string &s);

@@ -362,7 +362,9 @@ std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why) {
   const bool bwd = p.dir > 0;
   const int64_t id = p.howmany > 1 ? p.idist : 0;
   const int64_t od = p.howmany > 1 ? p.odist : 0;
-  // 1. one fused kernel (the streaming unit-stride variant when it applies)
+  // 1. one fused kernel (along the members of a column layout, else the
+  // streaming unit-stride variant when it applies)
+  if (auto node = build_columns_node(p, why)) return node;
   Choice c;
   const bool packed = p.istride == 1 && p.ostride == 1 &&
                       (p.howmany <= 1 || (p.idist == p.n && p.odist == p.n));
@@ -378,6 +380,7 @@ std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why) {
     return node;
   }
   // 2. four-step over the most balanced split with kernels for both sides
+  if (auto node = build_tile_fourstep_node(p, why)) return node;
   int64_t best1 = 0;
   Choice bc, br;
   for (int64_t n1 = 2; n1 * n1 <= p.n * 4 && n1 < p.n; ++n1) {

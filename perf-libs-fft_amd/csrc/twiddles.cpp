@@ -10,20 +10,20 @@
 
 namespace plf {
 
-void unit_root(int64_t num, int64_t den, double *re, double *im) {
+void unit_root_l(int64_t num, int64_t den, long double *re, long double *im) {
   int64_t r = num % den;
   if (r < 0) r += den;
   // reduce to an angle in [0, pi/4] with exact integer arithmetic over 8*den
   __int128 D = (__int128)den * 8;
   __int128 t = (__int128)r * 8;
-  double ss = 1.0, cs = 1.0;
+  long double ss = 1.0L, cs = 1.0L;
   if (2 * t > D) {
     t = D - t;
-    ss = -1.0;
+    ss = -1.0L;
   }
   if (4 * t > D) {
     t = D / 2 - t;
-    cs = -1.0;
+    cs = -1.0L;
   }
   bool swap = false;
   if (8 * t > D) {
@@ -38,8 +38,15 @@ void unit_root(int64_t num, int64_t den, double *re, double *im) {
     c = s;
     s = tmp;
   }
-  *re = (double)(cs * c);
-  *im = (double)(ss * s);
+  *re = cs * c;
+  *im = ss * s;
+}
+
+void unit_root(int64_t num, int64_t den, double *re, double *im) {
+  long double c, s;
+  unit_root_l(num, den, &c, &s);
+  *re = (double)c;
+  *im = (double)s;
 }
 
 std::vector<double> stockham_twiddles(const std::vector<int> &chain) {
