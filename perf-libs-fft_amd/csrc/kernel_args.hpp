@@ -14,7 +14,11 @@ struct GenericDesc {
   int radix[kMaxStages];
   int L[kMaxStages];
   int twoff[kMaxStages];
+  uint32_t magic[kMaxStages];  // ceil(2^32 / L): b / L = umulhi(b, magic), b < 2^16, L > 1
 };
+inline uint32_t division_magic(int64_t L) {
+  return L > 1 ? (uint32_t)(((uint64_t(1) << 32) + (uint64_t)L - 1) / (uint64_t)L) : 0;
+}
 
 // One argument block for all kernels; each kernel documents the fields it
 // reads. Strides and distances count logical elements.

@@ -119,11 +119,13 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2c(KArgs a) {
   const int64_t is = a.istride, os = a.ostride;
   Eng::template run<false>(
       a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) {
-        cpx<C> v = ST::ld(in[(int64_t)e * is]);
+      [&](int b, int o) {
+        cpx<C> v = ST::ld(in[(int64_t)b * is + (int64_t)o * is]);
         return BWD ? cswap(v) : v;
       },
-      [&](int e, cpx<C> v) { out[(int64_t)e * os] = ST::st(BWD ? cswap(v) : v); });
+      [&](int b, int o, cpx<C> v) {
+        out[(int64_t)b * os + (int64_t)o * os] = ST::st(BWD ? cswap(v) : v);
+      });
 }
 
 // Batched C2C of a small odd prime N (3..23) with packed members (unit
@@ -172,26 +174,51 @@ __global__ void __launch_bounds__(256) k_c2c_staged(KArgs a) {
 // batched C2C, unit element stride: streaming (non-temporal) global access;
 // with a PAIR engine neighbouring elements of one thread merge into 16-byte
 // accesses.
+// Addresses are the block's base in scalar registers plus a 32-bit offset per
+// lane: TPB times the member distance stays below 4 GiB (build_c2c_node
+// checks).
 template <typename S, bool BWD, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_c2c_unit(KArgs a) {
+__device__ __forceinline__ void c2c_unit_body(const KArgs &a) {
   using ST = StorageT<S>;
   using E = typename ST::E;
   using C = typename Eng::C;
   constexpr int TPT = Eng::TPT;
-  const int g = threadIdx.x / TPT;
-  const int t = threadIdx.x % TPT;
-  const int64_t tr = (int64_t)blockIdx.x * TPB + g;
-  const bool valid = tr < a.count;
-  const E *in = static_cast<const E *>(a.in) + (valid ? tr * a.idist : 0);
-  E *out = static_cast<E *>(a.out) + (valid ? tr * a.odist : 0);
+  const int g = TPB == 1 ? 0 : threadIdx.x / TPT;
+  const int t = TPB == 1 ? threadIdx.x : threadIdx.x % TPT;
+  const int64_t tr0 = (int64_t)blockIdx.x * TPB;
+  const bool valid = TPB == 1 || tr0 + g < a.count;
+  const E *in = static_cast<const E *>(a.in) + tr0 * a.idist;
+  E *out = static_cast<E *>(a.out) + tr0 * a.odist;
+  const uint32_t gi = TPB == 1 || !valid ? 0 : g * (uint32_t)a.idist;
+  const uint32_t go = TPB == 1 || !valid ? 0 : g * (uint32_t)a.odist;
   cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  Eng::template run<false>(
-      a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) {
-        cpx<C> v = ST::ldnt(in + e);
-        return BWD ? cswap(v) : v;
-      },
-      [&](int e, cpx<C> v) { ST::stnt(out + e, BWD ? cswap(v) : v); });
+  const cpx<C> *tw = static_cast<const cpx<C> *>(a.tw);
+  if constexpr (Eng::REGS_IN) {
+    Eng::template run<false>(
+        a.desc, lds, tw, t, valid,
+        [&](int b, int o) {
+          cpx<C> v = ST::ldnt(&at_u32(in + o, gi + b));
+          return BWD ? cswap(v) : v;
+        },
+        [&](int b, int o, cpx<C> v) {
+          ST::stnt(const_cast<E *>(&at_u32(out + o, go + b)), BWD ? cswap(v) : v);
+        });
+  } else {  // PAIR: neighbouring elements through one pointer, so that they merge
+    const E *x = in + gi;
+    E *y = out + go;
+    Eng::template run<false>(
+        a.desc, lds, tw, t, valid,
+        [&](int e) {
+          cpx<C> v = ST::ldnt(x + e);
+          return BWD ? cswap(v) : v;
+        },
+        [&](int e, cpx<C> v) { ST::stnt(y + e, BWD ? cswap(v) : v); });
+  }
+}
+
+template <typename S, bool BWD, int TPB, class Eng>
+__global__ void __launch_bounds__(Eng::TPT *TPB) k_c2c_unit(KArgs a) {
+  c2c_unit_body<S, BWD, TPB, Eng>(a);
 }
 
 // k_c2c_unit with at least WAVES waves per SIMD: the register budget is cut
@@ -200,24 +227,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2c_unit(KArgs a) {
 template <typename S, bool BWD, int TPB, class Eng, int WAVES>
 __global__ void __launch_bounds__(Eng::TPT *TPB) __attribute__((amdgpu_waves_per_eu(WAVES)))
 k_c2c_unit_occ(KArgs a) {
-  using ST = StorageT<S>;
-  using E = typename ST::E;
-  using C = typename Eng::C;
-  constexpr int TPT = Eng::TPT;
-  const int g = threadIdx.x / TPT;
-  const int t = threadIdx.x % TPT;
-  const int64_t tr = (int64_t)blockIdx.x * TPB + g;
-  const bool valid = tr < a.count;
-  const E *in = static_cast<const E *>(a.in) + (valid ? tr * a.idist : 0);
-  E *out = static_cast<E *>(a.out) + (valid ? tr * a.odist : 0);
-  cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  Eng::template run<false>(
-      a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) {
-        cpx<C> v = ST::ldnt(in + e);
-        return BWD ? cswap(v) : v;
-      },
-      [&](int e, cpx<C> v) { ST::stnt(out + e, BWD ? cswap(v) : v); });
+  c2c_unit_body<S, BWD, TPB, Eng>(a);
 }
 
 // batched C2C, unit element stride, software-pipelined: a block walks the

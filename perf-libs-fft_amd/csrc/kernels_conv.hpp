@@ -34,16 +34,16 @@ struct ConvMid {
   static constexpr int NB0 = Ch::N / R0;
   static constexpr int KB0 = (NB0 + TPT - 1) / TPT;
   static constexpr int SLOTS = KB0 * R0;
-  static __device__ __forceinline__ bool act(int t, int k) {
-    return (NB0 % TPT == 0) || (t + k * TPT < NB0);
+  // butterfly of slot k (threads past the last one repeat it)
+  static __device__ __forceinline__ int bfly(int t, int k) {
+    const int b = t + k * TPT;
+    return (NB0 % TPT == 0 || b < NB0) ? b : NB0 - 1;
   }
-  static __device__ __forceinline__ void load_B(const cpx<C> *B, int t, bool valid,
-                                                cpx<C> (&bv)[SLOTS]) {
+  static __device__ __forceinline__ void load_B(const cpx<C> *B, int t, cpx<C> (&bv)[SLOTS]) {
 #pragma unroll
     for (int k = 0; k < KB0; ++k)
 #pragma unroll
-      for (int m = 0; m < R0; ++m)
-        bv[k * R0 + m] = (act(t, k) && valid) ? B[t + k * TPT + m * NB0] : cpx<C>{C(0), C(0)};
+      for (int m = 0; m < R0; ++m) bv[k * R0 + m] = B[bfly(t, k) + m * NB0];
   }
   template <class First>
   static __device__ __forceinline__ void gather(const cpx<C> *lds, int t,
@@ -53,8 +53,7 @@ struct ConvMid {
     for (int k = 0; k < KB0; ++k)
 #pragma unroll
       for (int m = 0; m < R0; ++m) {
-        const cpx<C> A = act(t, k) ? lds[lds_pad<Eng::PAD>(t + k * TPT + m * NB0)]
-                                   : cpx<C>{C(0), C(0)};
+        const cpx<C> A = lds[lds_pad<Eng::PAD>(bfly(t, k) + m * NB0)];
         if (k == 0 && m == 0 && t == 0) first(A);
         vin[k * R0 + m] = cswap(cmul(A, bv[k * R0 + m]));
       }
@@ -86,11 +85,15 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_bluestein(KArgs a) {
   const cpx<C> *B = static_cast<const cpx<C> *>(a.aux0) + (mt ? rec->B_off : 0);
   const cpx<C> *chirp = static_cast<const cpx<C> *>(a.aux1) + (mt ? rec->chirp_off : 0);
   const int64_t is = mt ? 1 : a.istride, os = mt ? rec->ostride : a.ostride;
-  auto load = [&](int e) {
-    if (e >= n) return cpx<C>{C(0), C(0)};
+  // zero padding: skipped where it is all padding (o >= n, the same for
+  // every thread), otherwise selected after a load of element 0
+  auto load = [&](int b, int o) {
+    if (o >= n) return cpx<C>{C(0), C(0)};
+    const int e = b + o < n ? b + o : 0;
     cpx<C> v = ST::ld(in[(int64_t)e * is]);
     if (BWD) v = cswap(v);
-    return cmul(v, chirp[e]);
+    v = cmul(v, chirp[e]);
+    return cpx<C>{b + o < n ? v.x : C(0), b + o < n ? v.y : C(0)};
   };
   auto store = [&](int e, cpx<C> v) {
     if (e < n) {
@@ -101,7 +104,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_bluestein(KArgs a) {
   if constexpr (Eng::NFIX > 0) {
     using Mid = ConvMid<Eng>;
     cpx<C> bv[Mid::SLOTS], vin[Mid::SLOTS];
-    Mid::load_B(B, t, valid, bv);
+    Mid::load_B(B, t, bv);
     Eng::template run<true>(a.desc, lds, tw, t, valid, load, [&](int, cpx<C>) {});
     Mid::gather(lds, t, bv, vin, [](cpx<C>) {});
     __syncthreads();  // the second transform's first exchange rewrites LDS

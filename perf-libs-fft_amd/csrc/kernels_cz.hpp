@@ -60,11 +60,14 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_col_in(KArgs a) {
   cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
   Eng::template run<false>(
       a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) {
-        const int64_t j = c2 + n2 * e;
-        if (j >= nn) return cpx<C>{C(0), C(0)};  // zero padding
+      [&](int b, int o) {
+        // zero padding: skipped where it is all padding (the same for every
+        // thread), otherwise selected after a load of element 0
+        if (n2 * o >= nn) return cpx<C>{C(0), C(0)};
+        const int64_t j0 = c2 + n2 * (b + o), j = j0 < nn ? j0 : 0;
         cpx<C> v = ST::ld(in[j * is]);
-        return cmul(BWD ? cswap(v) : v, chirp[j]);
+        v = cmul(BWD ? cswap(v) : v, chirp[j]);
+        return cpx<C>{j0 < nn ? v.x : C(0), j0 < nn ? v.y : C(0)};
       },
       [&](int k1, cpx<C> v) { ws[(int64_t)k1 * n2] = cmul(v, cz_twiddle(split, shift, c2 * k1)); });
 }
@@ -102,9 +105,8 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_row_mid(KArgs a) {
   for (int k = 0; k < KB0; ++k)
 #pragma unroll
     for (int m = 0; m < R0; ++m) {
-      const int b = t + k * TPT;
-      const bool act = (NB0 % TPT == 0) || (b < NB0);
-      bv[k * R0 + m] = (act && valid) ? Brow[b + m * NB0] : cpx<C>{C(0), C(0)};
+      const int b = (NB0 % TPT == 0 || t + k * TPT < NB0) ? t + k * TPT : NB0 - 1;
+      bv[k * R0 + m] = Brow[b + m * NB0];
     }
   Eng::template run<true>(
       a.desc, lds, tw, t, valid, [&](int e) { return rowp[e]; }, [&](int, cpx<C>) {});
@@ -112,10 +114,8 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_row_mid(KArgs a) {
   for (int k = 0; k < KBL; ++k)
 #pragma unroll
     for (int m = 0; m < RL; ++m) {
-      const int b = t + k * TPT;
-      const bool act = (NBL % TPT == 0) || (b < NBL);
-      wv[k * RL + m] = (act && valid) ? cz_twiddle(split, shift, k1 * (b + m * NBL))
-                                      : cpx<C>{C(0), C(0)};
+      const int b = (NBL % TPT == 0 || t + k * TPT < NBL) ? t + k * TPT : NBL - 1;
+      wv[k * RL + m] = cz_twiddle(split, shift, k1 * (b + m * NBL));
     }
   // Rader (aux3 set): bin 0 of the forward transform, A_0 = sum of the
   // permuted inputs, goes to the member's slot for X_0 = x_0 + A_0
@@ -125,9 +125,8 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_row_mid(KArgs a) {
   for (int k = 0; k < KB0; ++k)
 #pragma unroll
     for (int m = 0; m < R0; ++m) {
-      const int b = t + k * TPT;
-      const bool act = (NB0 % TPT == 0) || (b < NB0);
-      const cpx<C> A = act ? lds[lds_pad<Eng::PAD>(b + m * NB0)] : cpx<C>{C(0), C(0)};
+      const int b = (NB0 % TPT == 0 || t + k * TPT < NB0) ? t + k * TPT : NB0 - 1;
+      const cpx<C> A = lds[lds_pad<Eng::PAD>(b + m * NB0)];
       if (k == 0 && m == 0 && slot && valid && k1 == 0 && t == 0) slot[2 * bi + 1] = A;
       vin[k * R0 + m] = cswap(cmul(A, bv[k * R0 + m]));
     }

@@ -28,6 +28,8 @@ void register_kernels_f32_unit(std::vector<KEntry> &r) {
   PLF_UNIT(S, P,   8,  32, 4, true,  16, 16);
   PLF_UNIT(S, P,  64,   4, 4, false, 16, 16, 4);
   PLF_UNIT(S, P,  32,   8, 4, true,  16, 16, 4);
+  // 2048: 52 us for 2^24 points; the paired 8-point chain 105
+  PLF_UNIT(S, P, 128,   2, 4, false, 16, 16, 8);
   PLF_UNIT(S, P, 128,   2, 4, true,  8, 8, 8, 4);
   // 4096: the first entry is the ESTIMATE choice and the incumbent of a timed
   // race; at 2^27 points the p5/p4 plain-exchange kernels measured 0.70 of

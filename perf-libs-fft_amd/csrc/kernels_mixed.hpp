@@ -100,8 +100,9 @@ struct MixedExec {
     const cpx<C> *aux = static_cast<const cpx<C> *>(a.aux);
     cpx<C> *ws = static_cast<cpx<C> *>(a.ws) + x.ws_off;
     const E *in = static_cast<const E *>(a.in) + x.in_off;
+    const E *src = in + (valid ? col : first);  // lanes past the tile read its first column
     EngT::template run<false>(
-        d, lds, tw, t, valid, [&](int e) { return io(a, ST::ld(in[col + (int64_t)e * n2])); },
+        d, lds, tw, t, valid, [&](int e) { return io(a, ST::ld(src[(int64_t)e * n2])); },
         [&](int k1, cpx<C> v) {
           // kind 4: the rows run on the Bluestein kernel, which swaps its
           // input again for a backward transform

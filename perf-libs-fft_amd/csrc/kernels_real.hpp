@@ -88,13 +88,17 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
       const int k = t + i * TPT;
       wk[i] = (2 * k <= NF) ? W[k] : cpx<C>{C(0), C(0)};
     }
-    auto body = [&](auto unit) {
+    auto body = [&](auto pair, auto unit) {
       constexpr bool U = decltype(unit)::value;
       Eng::template run<true>(
           a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-          [&](int e) {
-            if constexpr (U) return ST::ld(reinterpret_cast<const E *>(x)[e]);
-            else return load_pair<ST>(x, e, is, pair_ok);
+          [&](int b, int o) {
+            if constexpr (decltype(pair)::value) {
+              return ST::ld(reinterpret_cast<const E *>(x)[b + o]);
+            } else {
+              const Rs *p = x + (int64_t)(2 * b) * is + (int64_t)(2 * o) * is;
+              return cpx<C>{ST::ldr(p[0]), ST::ldr(p[is])};
+            }
           },
           [&](int, cpx<C>) {});
       if (!valid) return;
@@ -104,8 +108,9 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
         if (2 * k <= NF) post(k, wk[i], U ? int64_t(1) : os);
       }
     };
-    if (pair_ok && os == 1) body(std::true_type{});
-    else body(std::false_type{});
+    if (pair_ok && os == 1) body(std::true_type{}, std::true_type{});
+    else if (pair_ok) body(std::true_type{}, std::false_type{});
+    else body(std::false_type{}, std::false_type{});
   } else {
     Eng::template run<true>(
         a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
@@ -256,15 +261,10 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even_split(KArgs a) {
       const int lo = t + q * TPT;
       const int hi = lo == 0 ? NB / 2 : NB - lo;
       cpx<C> xl[R0], xh[R0];
-      if (valid) {
 #pragma unroll
-        for (int j = 0; j < R0; ++j) {
-          xl[j] = ld(lo + j * NB);
-          xh[j] = ld(hi + j * NB);
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < R0; ++j) xl[j] = xh[j] = cpx<C>{C(0), C(0)};
+      for (int j = 0; j < R0; ++j) {
+        xl[j] = ld(lo + j * NB);
+        xh[j] = ld(hi + j * NB);
       }
       // each pair of loaded values feeds two outputs, so the inputs can be
       // overwritten as the outputs are formed
@@ -282,7 +282,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even_split(KArgs a) {
           vh[R0 - 1 - j] = pre(B, A, mul_wc<2 * R0, R0 - 1 - j>(whi), false);
         });
       } else {
-        const cpx<C> xm = valid ? ld(M) : cpx<C>{C(0), C(0)};  // X[m] pairs with X[0]
+        const cpx<C> xm = ld(M);  // X[m] pairs with X[0]
         vl[0] = pre(xl[0], xm, cpx<C>{C(1), C(0)}, true);
         static_for<R0 / 2 + 1>([&](auto J) {
           constexpr int j = decltype(J)::value;
@@ -321,8 +321,16 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even_split(KArgs a) {
 // C2R, even n = 2m. flags bit0: reals may be written in pairs.
 // aux0: W_n^k, k = 0..m-1 (forward sign; conjugated here).
 // ---------------------------------------------------------------------------
+// The register cap keeps the scheduler from holding all of a thread's 2 R0
+// bins before the first is used (98 registers for 16 x 16, where 57 do).
+template <typename S, class Eng>
+constexpr int c2r_waves() {
+  if (sizeof(typename Eng::C) == 8) return Eng::NFIX > 0 ? 3 : 2;
+  return Eng::NFIX > 0 ? 6 : 4;
+}
 template <typename S, bool UNUSED, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even(KArgs a) {
+__global__ void __launch_bounds__(Eng::TPT *TPB)
+    __attribute__((amdgpu_waves_per_eu(c2r_waves<S, Eng>()))) k_c2r_even(KArgs a) {
   using ST = StorageT<S>;
   using E = typename ST::E;
   using Rs = typename ST::Rs;
@@ -382,14 +390,13 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even(KArgs a) {
       constexpr bool U = decltype(unit)::value;  // unit input stride
 #pragma unroll
       for (int k = 0; k < KB; ++k) {
-        const int b = t + k * TPT;
-        const bool act = valid && ((NB % TPT == 0) || (b < NB));
-        const cpx<C> wb = act ? W[b] : cpx<C>{C(1), C(0)};
+        int b = t + k * TPT;
+        if (NB % TPT != 0) b = b < NB ? b : NB - 1;
+        const cpx<C> wb = W[b];
 #pragma unroll
         for (int j = 0; j < R0; ++j)
-          vin[k * R0 + j] = act ? pre(b + j * NB, j == 0 ? wb : cmul(wb, W[j * NB]),
-                                      U ? int64_t(1) : is)
-                                : cpx<C>{C(0), C(0)};
+          vin[k * R0 + j] =
+              pre(b + j * NB, j == 0 ? wb : cmul(wb, W[j * NB]), U ? int64_t(1) : is);
       }
     };
     if (is == 1) build(std::true_type{});
@@ -692,23 +699,19 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_dct3_even(KArgs a) {
     cpx<C> vin[KB * R0];
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
-      const int b = t + k * TPT;
-      const bool act = valid && ((NB % TPT == 0) || (b < NB));
-      const cpx<C> Wb = act ? W[b] : cpx<C>{C(1), C(0)};
-      const cpx<C> wb = act ? w[b] : cpx<C>{C(1), C(0)};
+      int b = t + k * TPT;
+      if (NB % TPT != 0) b = b < NB ? b : NB - 1;
+      const cpx<C> Wb = W[b], wb = w[b];
 #pragma unroll
       for (int j = 0; j < R0; ++j) {
         const int e = b + j * NB;
         const cpx<C> We = j == 0 ? Wb : cmul(Wb, W[j * NB]);
         const cpx<C> we = j == 0 ? wb : cmul(wb, w[j * NB]);
         const cpx<C> wme = cconj_mul(wm, we);
-        if (act) {
-          const cpx<C> A = cconj_mul(cpx<C>{lu[e], e == 0 ? C(0) : -lu[n - e]}, we);
-          const cpx<C> B = cconj_mul(cpx<C>{lu[NF - e], -lu[NF + e]}, wme);
-          vin[k * R0 + j] = z(A, B, We);
-        } else {
-          vin[k * R0 + j] = cpx<C>{C(0), C(0)};
-        }
+        const C un = lu[e == 0 ? 0 : n - e];
+        const cpx<C> A = cconj_mul(cpx<C>{lu[e], e == 0 ? C(0) : -un}, we);
+        const cpx<C> B = cconj_mul(cpx<C>{lu[NF - e], -lu[NF + e]}, wme);
+        vin[k * R0 + j] = z(A, B, We);
       }
     }
     __syncthreads();  // u is read; stage 0 overwrites the LDS

@@ -281,6 +281,7 @@ std::unique_ptr<MixedPlan> MixedPlan::build(int prec, int fixed_bits, int dir, i
       d.radix[s] = ch[s];
       d.L[s] = (int)L;
       d.twoff[s] = (int)off;
+      d.magic[s] = division_magic(L);
       if (s > 0) off += L * (ch[s] - 1);
       L *= ch[s];
     }

@@ -178,6 +178,7 @@ hipError_t EngineData::init(const Choice &c, int64_t len) {
       d.radix[s] = c.chain[s];
       d.L[s] = (int)L;
       d.twoff[s] = (int)off;
+      d.magic[s] = division_magic(L);
       if (s > 0) off += L * (c.chain[s] - 1);
       L *= c.chain[s];
     }
@@ -369,6 +370,10 @@ std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why) {
   const bool packed = p.istride == 1 && p.ostride == 1 &&
                       (p.howmany <= 1 || (p.idist == p.n && p.odist == p.n));
   if (p.istride == 1 && p.ostride == 1) c = choose(KK_C2C_UNIT, p.n, p.prec, bwd, 0, packed);
+  // the unit-stride kernels address a block's members with 32-bit offsets
+  if (c.e && c.e->tpb > 1 &&
+      std::max(id, od) >= (int64_t(1) << 32) / c.e->tpb / (2 * prec_real_bytes(p.prec)) - p.n)
+    c = Choice();
   if (!c.e) c = choose(KK_C2C, p.n, p.prec, bwd);
   if (c.e) {
     auto node = std::make_unique<BatchC2CNode>(c, p.n, p.howmany, p.istride, id, p.ostride, od);
