@@ -1,0 +1,25 @@
+// flex_chain.hpp -- choice of a flexible chain (flex_engine.hpp).
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <vector>
+
+#include "flex_args.hpp"
+
+namespace plf {
+
+// The chain, thread count and LDS layout for members of length n (2 <= n <
+// 2^15) at up to `pts` points per thread and `block` threads per block, with
+// elements of `csize` bytes: least predicted cost, LDS up to `lds_max` bytes.
+// False if n has a prime factor above 13 or does not fit.
+// lanes > 0: that many neighbouring members per row of threads (members
+// closer together than their elements), or fewer if they do not fit.
+bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int lanes,
+                 FlexDesc *out);
+std::vector<int> flex_radices(const FlexDesc &d);
+inline int flex_threads(const FlexDesc &d) { return (d.tpt * d.tpb + 63) / 64 * 64; }
+inline size_t flex_lds(const FlexDesc &d, int csize) { return (size_t)d.tpb * d.lper * csize; }
+
+}  // namespace plf

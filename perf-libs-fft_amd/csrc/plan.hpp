@@ -85,6 +85,8 @@ std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why);
 // they do not apply
 std::unique_ptr<Node> build_columns_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_tile_fourstep_node(const Problem &p, std::string *why);
+// Lengths without a compiled chain (flex_plan.cpp), likewise
+std::unique_ptr<Node> build_flex_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_real_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_r2r_node(const Problem &p, std::string *why);
 // Q0.15 / Q0.7 problems (p.fixed_bits != 0): power-of-two n only.

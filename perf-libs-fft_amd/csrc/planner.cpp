@@ -375,6 +375,9 @@ std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why) {
       std::max(id, od) >= (int64_t(1) << 32) / c.e->tpb / (2 * prec_real_bytes(p.prec)) - p.n)
     c = Choice();
   if (!c.e) c = choose(KK_C2C, p.n, p.prec, bwd);
+  if (!c.e || c.e->n == 0) {
+    if (auto node = build_flex_node(p, why)) return node;
+  }
   if (c.e) {
     auto node = std::make_unique<BatchC2CNode>(c, p.n, p.howmany, p.istride, id, p.ostride, od);
     hipError_t err = node->init();

@@ -315,6 +315,9 @@ std::unique_ptr<Node> build_real_node(const Problem &p, std::string *why) {
   if (p.n % 2 == 0) {
     c = choose(r2c ? KK_R2C_E : KK_C2R_E, p.n / 2, p.prec, false);
     half = c.e != nullptr;
+    if (!c.e || c.e->n == 0) {
+      if (auto node = build_flex_node(p, why)) return node;
+    }
   }
   if (!c.e && p.n % 2 == 0 && p.n >= 8) {
     // packed half-length transform on the four-step passes
@@ -595,6 +598,9 @@ std::unique_ptr<Node> build_r2r_node(const Problem &p, std::string *why) {
   if (p.n % 2 == 0) {
     c = choose(two ? KK_DCT2_E : KK_DCT3_E, p.n / 2, p.prec, dst);
     half = c.e != nullptr;
+    if (!c.e || c.e->n == 0) {
+      if (auto node = build_flex_node(p, why)) return node;
+    }
   }
   if (!c.e) c = choose(two ? KK_DCT2_F : KK_DCT3_F, p.n, p.prec, dst);
   if (!c.e) {
