@@ -51,7 +51,10 @@ struct FlexEngine {
         q[k] = b;
         j[k] = 0;
 #pragma unroll
-        for (int m = 0; m < R; ++m) v[k][m] = load(b, m * NB);
+        for (int m = 0; m < R; ++m) {
+          v[k][m] = load(b, m * NB);
+          burst_after<Load>(v[k], m);
+        }
       } else {
         q[k] = (int)__umulhi((uint32_t)b, s.magic);
         j[k] = b - q[k] * L;

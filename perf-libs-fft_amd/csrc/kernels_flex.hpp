@@ -137,7 +137,7 @@ __global__ void __launch_bounds__(BLOCK) k_flex_c2r(FlexArgs f) {
   FlexEngine<C, false>::run(
       *f.d, dyn_lds<C>() + th.g * f.d->lper, static_cast<const cpx<C> *>(a.tw), th.t, th.live,
       valid,
-      [&](int b, int o) {
+      in_bursts<4>([&](int b, int o) {
         const int e = b + o;
         cpx<C> A = ST::ld(at_u32(X + (int64_t)o * is, gi + b * is));
         cpx<C> B = ST::ld(at_u32(X, gi + (m - e) * is));
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(BLOCK) k_flex_c2r(FlexArgs f) {
         const cpx<C> d = {A.x - B.x, A.y + B.y};        // A - conj B
         const cpx<C> wd = cconj_mul(d, at_u32(W + o, b));  // W^{-e} (A - conj B)
         return cswap(cpx<C>{s.x - wd.y, s.y + wd.x});   // s + i wd, swapped
-      },
+      }),
       [&](int b, int o, cpx<C> v) {
         v = cswap(v);
         const int e = b + o;
@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(BLOCK) k_flex_dct3(FlexArgs f) {
   __syncthreads();
   FlexEngine<C, true, true>::run(
       *f.d, lds, static_cast<const cpx<C> *>(a.tw), t, th.live, valid,
-      [&](int b, int o) {
+      in_bursts<2>([&](int b, int o) {
         const int e = b + o;
         // X_e and X_{m-e}: (u_k - i u_{n-k}) conj(w_k), u_n = 0
         const C un = lu[e == 0 ? 0 : n - e];
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(BLOCK) k_flex_dct3(FlexArgs f) {
         const cpx<C> sm = {A.x + B.x, A.y - B.y}, d = {A.x - B.x, A.y + B.y};
         const cpx<C> wd = cconj_mul(d, at_u32(W + o, b));
         return cswap(cpx<C>{sm.x - wd.y, sm.y + wd.x});
-      },
+      }),
       [](int, int, cpx<C>) {});
   if (!valid || !th.live) return;
   // swap(lds[e]) = v_{2e} + i v_{2e+1}; y[o] = v_i, i = o/2 (o even) or

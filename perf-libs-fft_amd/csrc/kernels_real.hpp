@@ -321,12 +321,13 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even_split(KArgs a) {
 // C2R, even n = 2m. flags bit0: reals may be written in pairs.
 // aux0: W_n^k, k = 0..m-1 (forward sign; conjugated here).
 // ---------------------------------------------------------------------------
-// The register cap keeps the scheduler from holding all of a thread's 2 R0
-// bins before the first is used (98 registers for 16 x 16, where 57 do).
+// Compile-time chains: a register cap keeps the scheduler from holding all of a
+// thread's 2 R0 bins before the first is used (98 registers for 16 x 16 in
+// FP32, where 57 do); loads in bursts of four cost the long chains 3 to 6 %.
 template <typename S, class Eng>
 constexpr int c2r_waves() {
-  if (sizeof(typename Eng::C) == 8) return Eng::NFIX > 0 ? 3 : 2;
-  return Eng::NFIX > 0 ? 6 : 4;
+  if (Eng::NFIX == 0) return 1;
+  return std::is_same_v<S, double> ? 3 : std::is_same_v<S, float> ? 6 : 5;
 }
 template <typename S, bool UNUSED, int TPB, class Eng>
 __global__ void __launch_bounds__(Eng::TPT *TPB)
@@ -405,7 +406,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB)
   } else {
     Eng::template run<false>(
         a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-        [&](int e) { return pre(e, W[e], is); }, store);
+        in_bursts<4>([&](int e) { return pre(e, W[e], is); }), store);
   }
 }
 
@@ -725,7 +726,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_dct3_even(KArgs a) {
     };
     Eng::template run<true>(
         a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-        [&](int e) { return z(X(e), X(m - e), W[e]); }, [&](int, cpx<C>) {});
+        in_bursts<2>([&](int e) { return z(X(e), X(m - e), W[e]); }), [&](int, cpx<C>) {});
   }
   if (!valid) return;
   // swap(lds[e]) = v_{2e} + i v_{2e+1}; coalesced stores y[o] = v_i with
@@ -763,11 +764,11 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_dct3_full(KArgs a) {
   const C s0 = (a.flags & 2) ? C(2) : C(1);
   Eng::template run<false>(
       a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int k) {
+      in_bursts<4>([&](int k) {
         const C ur = dct3_in<ST, DST>(x, k, n, is, s0);
         const C ui = k == 0 ? C(0) : -dct3_in<ST, DST>(x, n - k, n, is, s0);
         return cswap(cconj_mul(cpx<C>{ur, ui}, w[k]));
-      },
+      }),
       [&](int i, cpx<C> v) {
         const int o = 2 * i < n ? 2 * i : 2 * (n - i) - 1;
         const C r = v.y;  // Re of swap(v)

@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_col_c2r(KArgs a) {
   const C hw = (a.flags & 2) ? C(0.5) : C(1);  // adjoint of R2C: interior bins halved
   Eng::template run<false>(
       a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) {
+      in_bursts<4>([&](int e) {
         const int64_t j = c2 + (int64_t)e * n2;
         cpx<C> A = ST::ld(X[j * is]);
         cpx<C> B = ST::ld(X[(M - j) * is]);
@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_col_c2r(KArgs a) {
         const cpx<C> d = {A.x - B.x, A.y + B.y};  // A - conj B
         const cpx<C> wd = cconj_mul(d, packed_twiddle(wn, j, shift2));  // W_n^{-j} d
         return cswap(cpx<C>{s.x - wd.y, s.y + wd.x});  // s + i wd, swapped: inverse DFT
-      },
+      }),
       [&](int k1, cpx<C> v) {
         ws[(int64_t)k1 * n2] = cmul(v, packed_twiddle(wm, c2 * (int64_t)k1, shift));
       });
