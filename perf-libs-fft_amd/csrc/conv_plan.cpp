@@ -102,6 +102,24 @@ static hipError_t bluestein_kernel(int64_t n, int64_t M, const std::vector<doubl
   return dft_f64_gpu(*B, M, 1);
 }
 
+std::vector<double> cz_mid_twiddles(int64_t n1, const Choice &mid) {
+  const int64_t n2 = mid.e->n, R = mid.chain[0], NB = n2 / R, M = n1 * n2;
+  std::vector<double> t;
+  t.reserve(2 * (size_t)(n1 * (NB + R)));
+  auto table = [&](int64_t count, int64_t step) {  // W_M^{k1 step i}, i < count
+    for (int64_t k1 = 0; k1 < n1; ++k1)
+      for (int64_t i = 0; i < count; ++i) {
+        double re, im;
+        unit_root(k1 * step * i % M, M, &re, &im);
+        t.push_back(re);
+        t.push_back(-im);
+      }
+  };
+  table(NB, 1);
+  table(R, NB);
+  return t;
+}
+
 // ---------------------------------------------------------------------------
 class FusedConvNode : public Node {
  public:
@@ -291,6 +309,7 @@ class ChirpZ3Node : public Node {
       sp.push_back(-im);
     }
     err = upload_table(split_, sp, prec_);
+    if (err == hipSuccess) err = upload_table(tmid_, cz_mid_twiddles(n1_, cmid_), prec_);
     if (err != hipSuccess) return err;
     std::vector<double> c = chirp_table(n_), B;
     err = bluestein_kernel(n_, M, c, &B);
@@ -344,12 +363,11 @@ class ChirpZ3Node : public Node {
       // 2. rows: DFT_n2, x B, the inverse's first DFT_n2
       if (err == hipSuccess) {
         a.tw = emid_.tw.p;
-        a.desc = emid_.d();
+        a.aux0 = tmid_.p;
         a.aux1 = B_.p;
         a.n = n2_;
         a.count = cb * n1_;
-        err = cmid_.e->launch(a, (a.count + cmid_.e->tpb - 1) / cmid_.e->tpb,
-                              cmid_.e->lds_bytes(n2_), s);
+        err = cmid_.e->launch(a, a.count / cmid_.e->tpb, cmid_.e->lds_bytes(n2_), s);
       }
       // 3. chirp-out columns
       if (err == hipSuccess) {
@@ -385,7 +403,7 @@ class ChirpZ3Node : public Node {
   Choice cin_, cmid_, cout_;
   EngineData ein_, emid_, eout_;
   int shift_ = 0;
-  DevMem split_, B_, c_;
+  DevMem split_, tmid_, B_, c_;
 };
 
 // Rader for a prime n in three passes over N = n - 1 = n1 * n2
@@ -426,6 +444,7 @@ class Rader3Node : public Node {
       sp.push_back(-im);
     }
     err = upload_table(split_, sp, prec_);
+    if (err == hipSuccess) err = upload_table(tmid_, cz_mid_twiddles(n1_, cmid_), prec_);
     if (err != hipSuccess) return err;
     gen_ = group_generator(n_);
     if (!gen_) return hipErrorInvalidValue;
@@ -495,12 +514,11 @@ class Rader3Node : public Node {
       if (err == hipSuccess) {
         a.in = nullptr;
         a.tw = emid_.tw.p;
-        a.desc = emid_.d();
+        a.aux0 = tmid_.p;
         a.aux1 = B_.p;
         a.n = n2_;
         a.count = nb * n1_;
-        err = cmid_.e->launch(a, (a.count + cmid_.e->tpb - 1) / cmid_.e->tpb,
-                              cmid_.e->lds_bytes(n2_), s);
+        err = cmid_.e->launch(a, a.count / cmid_.e->tpb, cmid_.e->lds_bytes(n2_), s);
       }
       // 3. permuted-output columns, one block per CU: the scattered stores
       // of fewer members in flight stay in L2 until their lines fill
@@ -540,7 +558,7 @@ class Rader3Node : public Node {
   EngineData ein_, emid_, eout_;
   int shift_ = 0;
   int64_t gen_ = 0;
-  DevMem split_, B_, perm_;
+  DevMem split_, tmid_, B_, perm_;
 };
 
 // The most balanced split N = n1 * n2 (n1 a power of two) with compiled
@@ -554,7 +572,7 @@ static bool rd3_choice(int64_t N, int prec, bool bwd, int64_t *n1_out, Choice *c
     Choice ci = choose(KK_RD_COL_IN, n1, prec, bwd);
     Choice cm = choose(KK_CZ_ROW_MID, n2, prec, bwd);
     Choice co = choose(KK_RD_COL_OUT, n1, prec, bwd);
-    if (!ci.e || !cm.e || !co.e) continue;
+    if (!ci.e || !cm.e || !co.e || n1 % cm.e->tpb) continue;
     const double bal = std::fabs(std::log((double)n1 / (double)n2));
     if (bal < best) {
       best = bal;
@@ -584,7 +602,7 @@ bool cz3_choice(int64_t n, int prec, bool bwd, Cz3Choice *out) {
       Choice ci = choose(KK_CZ_COL_IN, n1, prec, bwd);
       Choice cm = choose(KK_CZ_ROW_MID, n2, prec, bwd);
       Choice co = choose(KK_CZ_COL_OUT, n1, prec, bwd);
-      if (!ci.e || !cm.e || !co.e) continue;
+      if (!ci.e || !cm.e || !co.e || n1 % cm.e->tpb) continue;
       out->M = M;
       out->n1 = n1;
       out->cin = ci;

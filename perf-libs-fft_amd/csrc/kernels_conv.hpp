@@ -16,49 +16,9 @@
 #pragma once
 
 #include "kernels.hpp"
+#include "tile_engine.hpp"
 
 namespace plf {
-
-// Between the two transforms of a static-chain engine: B is loaded before
-// the first transform at the slots where the second one's stage 0 takes its
-// inputs (butterfly b = t + k TPT, element b + m N / R0), and one LDS read
-// turns the first transform's natural-order output into those inputs,
-// times B and swapped; `first` sees element 0. The caller puts a barrier
-// after it and runs the second transform from registers.
-template <class Eng>
-struct ConvMid {
-  using C = typename Eng::C;
-  using Ch = typename Eng::Ch;
-  static constexpr int TPT = Eng::TPT;
-  static constexpr int R0 = Ch::radix(0);
-  static constexpr int NB0 = Ch::N / R0;
-  static constexpr int KB0 = (NB0 + TPT - 1) / TPT;
-  static constexpr int SLOTS = KB0 * R0;
-  // butterfly of slot k (threads past the last one repeat it)
-  static __device__ __forceinline__ int bfly(int t, int k) {
-    const int b = t + k * TPT;
-    return (NB0 % TPT == 0 || b < NB0) ? b : NB0 - 1;
-  }
-  static __device__ __forceinline__ void load_B(const cpx<C> *B, int t, cpx<C> (&bv)[SLOTS]) {
-#pragma unroll
-    for (int k = 0; k < KB0; ++k)
-#pragma unroll
-      for (int m = 0; m < R0; ++m) bv[k * R0 + m] = B[bfly(t, k) + m * NB0];
-  }
-  template <class First>
-  static __device__ __forceinline__ void gather(const cpx<C> *lds, int t,
-                                                const cpx<C> (&bv)[SLOTS], cpx<C> (&vin)[SLOTS],
-                                                First &&first) {
-#pragma unroll
-    for (int k = 0; k < KB0; ++k)
-#pragma unroll
-      for (int m = 0; m < R0; ++m) {
-        const cpx<C> A = lds[lds_pad<Eng::PAD>(bfly(t, k) + m * NB0)];
-        if (k == 0 && m == 0 && t == 0) first(A);
-        vin[k * R0 + m] = cswap(cmul(A, bv[k * R0 + m]));
-      }
-  }
-};
 
 // aux0: B (M entries), aux1: chirp c (n entries); a.n = M, a.n1 = n.
 // Gathered launch (aux2 = BlueMember records, one per transform; a mixed
@@ -101,24 +61,69 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_bluestein(KArgs a) {
       out[(int64_t)e * os] = ST::st(BWD ? cswap(r) : r);
     }
   };
-  if constexpr (Eng::NFIX > 0) {
-    using Mid = ConvMid<Eng>;
-    cpx<C> bv[Mid::SLOTS], vin[Mid::SLOTS];
-    Mid::load_B(B, t, bv);
-    Eng::template run<true>(a.desc, lds, tw, t, valid, load, [&](int, cpx<C>) {});
-    Mid::gather(lds, t, bv, vin, [](cpx<C>) {});
-    __syncthreads();  // the second transform's first exchange rewrites LDS
-    Eng::E::run_regs(vin, lds, tw, t, store, valid);
-  } else {
-    Eng::template run<true>(a.desc, lds, tw, t, valid, load, [&](int, cpx<C>) {});
-    for (int e = t; e < M; e += TPT) {
-      const int p = lds_pad<Eng::PAD>(e);
-      lds[p] = cswap(cmul(lds[p], B[e]));
-    }
-    __syncthreads();
-    Eng::template run<false, true>(
-        a.desc, lds, tw, t, valid, [&](int) { return cpx<C>{C(0), C(0)}; }, store);
+  Eng::template run<true>(a.desc, lds, tw, t, valid, load, [&](int, cpx<C>) {});
+  for (int e = t; e < M; e += TPT) {
+    const int p = lds_pad<Eng::PAD>(e);
+    lds[p] = cswap(cmul(lds[p], B[e]));
   }
+  __syncthreads();
+  Eng::template run<false, true>(
+      a.desc, lds, tw, t, valid, [&](int) { return cpx<C>{C(0), C(0)}; }, store);
+}
+
+// k_bluestein of a compile-time padded length on the two-transform tile engine
+// (ConvTile): TPB members of TPT threads. Bound by LDS latency and the two
+// transforms' arithmetic. FP64 members of 1399 (M = 4096, 5996 of them) 187
+// -> 144 us against the engine that passes the first transform's result
+// through LDS, FP32 members of 59 (M = 128, 280000) 140 -> 114 us.
+template <typename S, bool BWD, int TPB, int TPT, class Ch>
+__global__ void __launch_bounds__(TPT *TPB) k_bluestein_tile(KArgs a) {
+  using ST = StorageT<S>;
+  using E = typename ST::E;
+  using C = typename ST::C;
+  using T = ConvTile<C, TPB, TPT, Ch>;
+  constexpr int R0 = Ch::radix(0), NB0 = Ch::N / R0;
+  const int tid = threadIdx.x;
+  const int t = tid % TPT;
+  const int64_t tr = (int64_t)blockIdx.x * TPB + tid / TPT;
+  const bool valid = tr < a.count;
+  const BlueMember *mt = static_cast<const BlueMember *>(a.aux2);
+  const BlueMember *rec = mt ? mt + (valid ? tr : 0) : nullptr;
+  const int n = mt ? (int)rec->n : (int)a.n1;
+  const E *in = static_cast<const E *>(a.in) + (mt ? rec->in_off : valid ? tr * a.idist : 0);
+  E *out = static_cast<E *>(a.out) + (mt ? rec->out_off : valid ? tr * a.odist : 0);
+  const cpx<C> *B = static_cast<const cpx<C> *>(a.aux0) + (mt ? rec->B_off : 0) + t;
+  const cpx<C> *chirp = static_cast<const cpx<C> *>(a.aux1) + (mt ? rec->chirp_off : 0);
+  const int64_t is = mt ? 1 : a.istride, os = mt ? rec->ostride : a.ostride;
+  T::run(
+      reinterpret_cast<C *>(dyn_lds<C>()), static_cast<const cpx<C> *>(a.tw), tid,
+      [&](int b, int m) {
+        // n <= M / 2 + 1, as M >= 2n - 2: the upper half is padding; below it
+        // padding is selected after a load of element 0
+        if (2 * m * NB0 > Ch::N) return cpx<C>{C(0), C(0)};
+        const int o = b + m * NB0, e = o < n ? o : 0;
+        cpx<C> v = ST::ld(in[(int64_t)e * is]);
+        v = cmul(BWD ? cswap(v) : v, chirp[e]);
+        return cpx<C>{o < n ? v.x : C(0), o < n ? v.y : C(0)};
+      },
+      [&](cpx<C> (&v)[T::KB][T::R]) {
+#pragma unroll
+        for (int k = 0; k < T::KB; ++k)
+#pragma unroll
+          for (int m = 0; m < T::R; ++m) v[k][m] = cswap(cmul(v[k][m], B[k * TPT + m * T::NB]));
+      },
+      [&](int b, const cpx<C> (&v)[R0]) {
+        if (!valid) return;
+#pragma unroll
+        for (int m = 0; m < R0; ++m) {
+          if (2 * m * NB0 > Ch::N) continue;
+          const int e = b + m * NB0;
+          if (e < n) {
+            const cpx<C> r = cmul(cswap(v[m]), chirp[e]);
+            out[(int64_t)e * os] = ST::st(BWD ? cswap(r) : r);
+          }
+        }
+      });
 }
 
 // aux0: B (m entries), aux1: perm (int32, m entries); a.n = m, a.n1 = n.
@@ -160,8 +165,6 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_rader(KArgs a) {
       out[0] = ST::st(BWD ? cswap(y0) : y0);
     }
   };
-  // (the register-resident middle step of k_bluestein measured slower here:
-  // the Rader chains 4.8.3 and 16.3.3.7 are already register-bound)
   Eng::template run<true>(a.desc, lds, tw, t, valid, load, [&](int, cpx<C>) {});
   for (int e = t; e < m; e += TPT) {
     const int p = lds_pad<Eng::PAD>(e);

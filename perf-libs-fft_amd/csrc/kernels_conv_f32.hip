@@ -7,15 +7,15 @@ namespace plf {
 void register_kernels_conv_f32(std::vector<KEntry> &r) {
     using S = float;
     constexpr int P = P_F32;
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,    8,  32, 8, 8);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,    8,  32, 16, 8);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,   16,  16, 16, 16);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,   32,   8, 16, 16, 2);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,   64,   4, 16, 16, 4);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,  128,   2, 16, 16, 8);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,  256,   1, 16, 16, 16);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P,  512,   1, 16, 16, 16, 2);
-    PLF_STATIC(k_bluestein, KK_BLUE, S, P, 1024,   1, 16, 16, 16, 4);
+    PLF_BLUE_TILE(S, P,    8,  32, 8, 8);
+    PLF_BLUE_TILE(S, P,    8,  32, 16, 8);
+    PLF_BLUE_TILE(S, P,   16,  16, 16, 16);
+    PLF_BLUE_TILE(S, P,   32,   8, 16, 2, 16);
+    PLF_BLUE_TILE(S, P,   64,   4, 16, 4, 16);
+    PLF_BLUE_TILE(S, P,  128,   2, 16, 8, 16);
+    PLF_BLUE_TILE(S, P,  256,   1, 16, 16, 16);
+    PLF_BLUE_TILE(S, P,  512,   1, 16, 2, 16, 16);
+    PLF_BLUE_TILE(S, P, 1024,   1, 16, 4, 16, 16);
     PLF_DYNAMIC(k_bluestein, KK_BLUE, S, P,  64,   4, 16);
     PLF_DYNAMIC(k_bluestein, KK_BLUE, S, P, 256,   1, 16);
     PLF_DYNAMIC(k_bluestein, KK_BLUE, S, P, 1024,  1, 16);

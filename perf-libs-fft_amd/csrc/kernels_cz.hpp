@@ -11,7 +11,7 @@
 //   2. row k1: DFT_n2 gives A[k1 + n1 k2]; times B (stored row-major by k1),
 //      swapped; the inverse transform's four-step, taken with the sides
 //      exchanged, starts with a DFT_n2 over the same row, so it runs on the
-//      same LDS contents, is twiddled by W_M^{k1 m2} and written back in place;
+//      same registers, is twiddled by W_M^{k1 m2} and written back in place;
 //   3. column m2: DFT_n1 over k1 gives bin m = m2 + n2 m1; swapped back,
 //      times c_m, stored for m < n.
 // The backward transform is swap o forward o swap on the input and output.
@@ -20,7 +20,8 @@
 // table (lo: 2^shift entries, then hi), n = engine length, n1, n2 = the
 // sides, bigdist = the transform length n, count = columns (members * n2) or
 // rows (members * n1). Pass 1: in = input (storage type, istride, idist),
-// out = workspace, aux1 = chirp. Pass 2: out = workspace, aux1 = B. Pass 3:
+// out = workspace, aux1 = chirp. Pass 2: out = workspace, aux0 = its own
+// twiddles (k_cz_row_mid), aux1 = B. Pass 3:
 // in = workspace, out = output (ostride, odist), aux1 = chirp.
 // Gathered launch (aux2 = CzMember records, one per member of the launch;
 // the members of a mixed-length batch that share M): each member's length,
@@ -28,6 +29,7 @@
 #pragma once
 
 #include "kernels.hpp"
+#include "tile_engine.hpp"
 
 namespace plf {
 
@@ -72,75 +74,47 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_col_in(KArgs a) {
       [&](int k1, cpx<C> v) { ws[(int64_t)k1 * n2] = cmul(v, cz_twiddle(split, shift, c2 * k1)); });
 }
 
-// Row pass. B is loaded with the row, at the slots where the second
-// transform's stage 0 takes its inputs, and the W_M twiddles during the
-// second transform, at the slots where its last stage leaves its outputs
-// (registers, not LDS). Between the two transforms one LDS pass turns the
-// first's natural-order output into the second's stage-0 layout, applying
-// B and the swap on the way.
-template <typename S, bool BWD, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_row_mid(KArgs a) {
-  using C = typename Eng::C;
-  using Ch = typename Eng::Ch;
-  constexpr int TPT = Eng::TPT;
-  constexpr int N = Ch::N;
-  constexpr int R0 = Ch::radix(0), RL = Ch::radix(Ch::count - 1);
-  constexpr int NB0 = N / R0, NBL = N / RL;
-  constexpr int KB0 = (NB0 + TPT - 1) / TPT, KBL = (NBL + TPT - 1) / TPT;
-  const int g = threadIdx.x / TPT;
-  const int t = threadIdx.x % TPT;
-  const int64_t row = xcd_block(blockIdx.x, gridDim.x) * TPB + g;
-  const bool valid = row < a.count;
-  const int64_t n1 = a.n1, n2 = a.n2;
-  const int64_t bi = valid ? row / n1 : 0, k1 = valid ? row % n1 : 0;
+// Row pass, on the two-transform tile engine (ConvTile): W rows of TPT threads
+// (n1 % W == 0). aux0: T1[k1][b] = W_M^{k1 b} (b < N / R, R the chain's first
+// radix), then T2[k1][m] = W_M^{k1 m N / R}: the twiddle of output b + m N / R
+// is the product of an entry per thread and one that the row's threads share.
+// Storage types and directions do not matter to it. Rows of 256 of 512 members
+// of 65536 (268 MB each way): 206 -> 141 us against two transforms through LDS.
+template <typename C, int W, int TPT, class Ch>
+__global__ void __launch_bounds__(TPT *W) k_cz_row_mid(KArgs a) {
+  using T = ConvTile<C, W, TPT, Ch>;
+  constexpr int N = Ch::N, R0 = Ch::radix(0), NB0 = N / R0;
+  const int tid = threadIdx.x;
+  const int t = tid % TPT;
+  const uint32_t n1 = (uint32_t)a.n1, tpm = n1 / W;  // tiles per member
+  const uint32_t bx = (uint32_t)xcd_block(blockIdx.x, gridDim.x);
+  const uint32_t bi = bx / tpm, k1 = (bx % tpm) * W + tid / TPT;
   const CzMember *mt = static_cast<const CzMember *>(a.aux2);
-  cpx<C> *rowp = static_cast<cpx<C> *>(a.out) + (mt ? mt[bi].ws_off : bi * n1 * n2) + k1 * n2;
-  const cpx<C> *split = static_cast<const cpx<C> *>(a.aux0);
-  const cpx<C> *Brow = static_cast<const cpx<C> *>(a.aux1) + (mt ? mt[bi].B_off : 0) + k1 * n2;
-  const cpx<C> *tw = static_cast<const cpx<C> *>(a.tw);
-  const int shift = a.shift;
-  cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  cpx<C> bv[KB0 * R0], wv[KBL * RL];
-#pragma unroll
-  for (int k = 0; k < KB0; ++k)
-#pragma unroll
-    for (int m = 0; m < R0; ++m) {
-      const int b = (NB0 % TPT == 0 || t + k * TPT < NB0) ? t + k * TPT : NB0 - 1;
-      bv[k * R0 + m] = Brow[b + m * NB0];
-    }
-  Eng::template run<true>(
-      a.desc, lds, tw, t, valid, [&](int e) { return rowp[e]; }, [&](int, cpx<C>) {});
-#pragma unroll
-  for (int k = 0; k < KBL; ++k)
-#pragma unroll
-    for (int m = 0; m < RL; ++m) {
-      const int b = (NBL % TPT == 0 || t + k * TPT < NBL) ? t + k * TPT : NBL - 1;
-      wv[k * RL + m] = cz_twiddle(split, shift, k1 * (b + m * NBL));
-    }
+  cpx<C> *row = static_cast<cpx<C> *>(a.out) + (mt ? mt[bi].ws_off : (int64_t)bi * n1 * N) +
+                (int64_t)k1 * N;
+  const cpx<C> *B = static_cast<const cpx<C> *>(a.aux1) + (mt ? mt[bi].B_off : 0) +
+                    (int64_t)k1 * N + t;
+  const cpx<C> *t1 = static_cast<const cpx<C> *>(a.aux0) + (int64_t)k1 * NB0;
+  const cpx<C> *t2 = static_cast<const cpx<C> *>(a.aux0) + (int64_t)n1 * NB0 + (int64_t)k1 * R0;
   // Rader (aux3 set): bin 0 of the forward transform, A_0 = sum of the
   // permuted inputs, goes to the member's slot for X_0 = x_0 + A_0
   cpx<C> *slot = static_cast<cpx<C> *>(a.aux3);
-  cpx<C> vin[KB0 * R0];
+  T::run(
+      reinterpret_cast<C *>(dyn_lds<C>()), static_cast<const cpx<C> *>(a.tw), tid,
+      [&](int b, int m) { return row[b + m * NB0]; },
+      [&](cpx<C> (&v)[T::KB][T::R]) {
+        if (slot && k1 == 0 && t == 0) slot[2 * bi + 1] = v[0][0];
 #pragma unroll
-  for (int k = 0; k < KB0; ++k)
+        for (int k = 0; k < T::KB; ++k)
 #pragma unroll
-    for (int m = 0; m < R0; ++m) {
-      const int b = (NB0 % TPT == 0 || t + k * TPT < NB0) ? t + k * TPT : NB0 - 1;
-      const cpx<C> A = lds[lds_pad<Eng::PAD>(b + m * NB0)];
-      if (k == 0 && m == 0 && slot && valid && k1 == 0 && t == 0) slot[2 * bi + 1] = A;
-      vin[k * R0 + m] = cswap(cmul(A, bv[k * R0 + m]));
-    }
-  __syncthreads();  // the second transform's first exchange rewrites LDS
-  cpx<C> out[KBL * RL];
-  Eng::E::run_regs_keep(vin, lds, tw, t, out);
-  if (valid)
+          for (int m = 0; m < T::R; ++m) v[k][m] = cswap(cmul(v[k][m], B[k * TPT + m * T::NB]));
+      },
+      [&](int b, const cpx<C> (&v)[R0]) {
+        const cpx<C> wb = t1[b];
 #pragma unroll
-    for (int k = 0; k < KBL; ++k)
-#pragma unroll
-      for (int m = 0; m < RL; ++m) {
-        const int b = t + k * TPT;
-        if ((NBL % TPT == 0) || (b < NBL)) rowp[b + m * NBL] = cmul(out[k * RL + m], wv[k * RL + m]);
-      }
+        for (int m = 0; m < R0; ++m)
+          row[b + m * NB0] = cmul(v[m], m == 0 ? wb : cmul(wb, t2[m]));
+      });
 }
 
 template <typename S, bool BWD, int TPB, class Eng>

@@ -206,3 +206,28 @@ inline void add_entry(std::vector<KEntry> &r, int kind, int prec, int n,
       r[r.size() - i].lds_scalars = 1;                                                    \
     }                                                                                     \
   } while (0)
+
+// Two-transform tile kernels (ConvTile): K<S, BWD, TPB, TPT, Chain>; the row
+// pass of the three-pass convolutions is one kernel for all storage types of a
+// compute type and both directions.
+#define PLF_CONV_LDS(S, TPT, TPB, ...)                                                     \
+  for (int i_ = 1; i_ <= 2; ++i_)                                                          \
+  r[r.size() - i_].conv_lds = ::plf::ConvTile<typename ::plf::StorageT<S>::C, TPB, TPT,     \
+                                              ::plf::Chain<__VA_ARGS__>>::LDS_BYTES
+#define PLF_BLUE_TILE(S, PREC, TPT, TPB, ...)                                              \
+  do {                                                                                     \
+    using ChT = ::plf::Chain<__VA_ARGS__>;                                                 \
+    ::plf::add_entry(r, ::plf::KK_BLUE, PREC, ChT::N, {__VA_ARGS__}, TPT, TPB, 0, true,    \
+                     &::plf::launch_k<&::plf::k_bluestein_tile<S, false, TPB, TPT, ChT>, TPT * TPB>, \
+                     &::plf::launch_k<&::plf::k_bluestein_tile<S, true, TPB, TPT, ChT>, TPT * TPB>); \
+    PLF_CONV_LDS(S, TPT, TPB, __VA_ARGS__);                                                \
+  } while (0)
+#define PLF_CZ_MID(S, PREC, TPT, TPB, ...)                                                 \
+  do {                                                                                     \
+    using ChT = ::plf::Chain<__VA_ARGS__>;                                                 \
+    constexpr auto run = &::plf::launch_k<                                                 \
+        &::plf::k_cz_row_mid<typename ::plf::StorageT<S>::C, TPB, TPT, ChT>, TPT * TPB>;   \
+    ::plf::add_entry(r, ::plf::KK_CZ_ROW_MID, PREC, ChT::N, {__VA_ARGS__}, TPT, TPB, 0, true, \
+                     run, run);                                                            \
+    PLF_CONV_LDS(S, TPT, TPB, __VA_ARGS__);                                                \
+  } while (0)

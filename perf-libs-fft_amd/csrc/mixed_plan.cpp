@@ -504,6 +504,7 @@ std::unique_ptr<MixedPlan> MixedPlan::build(int prec, int fixed_bits, int dir, i
     g->shift = spl.second;
     hipError_t err = g->ein.init(g->cin, g->n1);
     if (err == hipSuccess) err = g->emid.init(g->cmid, g->n2);
+    if (err == hipSuccess) err = upload_table(g->tmid, cz_mid_twiddles(g->n1, g->cmid), prec);
     if (err == hipSuccess) err = g->eout.init(g->cout, g->n1);
     if (err == hipSuccess)
       err = g->members.upload(kv.second.data(), kv.second.size() * sizeof(CzMember));
@@ -643,10 +644,10 @@ hipError_t MixedPlan::enqueue(const void *in, void *out, void *ws, hipStream_t s
     // 2. rows (B tables in aux at the members' B offsets)
     if (err == hipSuccess) {
       k.tw = g->emid.tw.p;
+      k.aux0 = g->tmid.p;
       k.n = g->n2;
       k.count = g->count * g->n1;
-      err = g->cmid.e->launch(k, (k.count + g->cmid.e->tpb - 1) / g->cmid.e->tpb,
-                              g->cmid.e->lds_bytes(g->n2), s);
+      err = g->cmid.e->launch(k, k.count / g->cmid.e->tpb, g->cmid.e->lds_bytes(g->n2), s);
     }
     // 3. chirp-out columns
     if (err == hipSuccess) {

@@ -54,6 +54,7 @@ class MixedPlan {
     EngineData ein, emid, eout;
     int64_t n1 = 0, n2 = 0, count = 0, split_off = 0;
     int shift = 0;
+    DevMem tmid;     // the middle pass's twiddles
     DevMem members;  // CzMember records
   };
   std::vector<std::unique_ptr<CzGroup>> cz_groups_;

@@ -157,6 +157,8 @@ struct Cz3Choice {
   int64_t M = 0, n1 = 0;
   Choice cin, cmid, cout;
 };
+// The middle pass's twiddles (k_cz_row_mid: T1, then T2) for n1 rows.
+std::vector<double> cz_mid_twiddles(int64_t n1, const Choice &mid);
 bool cz3_choice(int64_t n, int prec, bool bwd, Cz3Choice *out);
 
 // Twiddle table of a Stockham radix chain, FORWARD sign, FP64:

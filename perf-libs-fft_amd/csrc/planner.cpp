@@ -168,7 +168,13 @@ hipError_t EngineData::init(const Choice &c, int64_t len) {
       const std::vector<uint16_t> t = mfma_dft16_table();
       return tw.upload(t.data(), t.size() * sizeof(uint16_t));
     }
-    hipError_t err = upload_table(tw, stockham_twiddles(c.chain), c.e->prec);
+    std::vector<double> t = stockham_twiddles(c.chain);
+    if (c.e->conv_lds) {
+      const std::vector<double> r =
+          stockham_twiddles(std::vector<int>(c.chain.rbegin(), c.chain.rend()));
+      t.insert(t.end(), r.begin(), r.end());
+    }
+    hipError_t err = upload_table(tw, t, c.e->prec);
     if (err != hipSuccess || c.e->n) return err;
     GenericDesc d{};
     d.n = (int)len;

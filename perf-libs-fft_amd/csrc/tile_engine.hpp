@@ -30,13 +30,26 @@ struct TileEngine {
   static constexpr int NS = Ch::count;
   static constexpr int BANKS = 256 / (int)sizeof(C);
   static constexpr int LPER = [] {
-    const int want = BANKS / 2 + (BANKS / 2 / W > 0 ? BANKS / 2 / W : 1);
+    const int want = (BANKS / 2 + (BANKS / 2 / W > 0 ? BANKS / 2 / W : 1)) % BANKS;
     int l = N + N / 16 + 1;
     while (l % BANKS != want) ++l;
     return l;
   }();
   static constexpr size_t LDS_BYTES = (size_t)W * LPER * sizeof(C);
   static_assert(NS >= 2, "one exchange at least");
+
+  // Map B alone, members within one wave: the exchange stays in the wave, whose
+  // LDS accesses are executed in order, so no barrier is needed.
+  static constexpr bool WAVE = !AIN && !AOUT && 64 % TPT == 0;
+  static __device__ __forceinline__ void sync() {
+    if constexpr (WAVE) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+      __syncthreads();
+    }
+  }
 
   template <int SI>
   struct St {
@@ -108,26 +121,29 @@ struct TileEngine {
                                               Store &store) {
     using T = St<SI>;
     compute<SI>(v, tw, tid);
-    if constexpr (SI == NS - 1) {
+    if constexpr (SI == NS - 1 && std::is_invocable_v<Store &, decltype(v)>) {
+      store(v);
+    } else if constexpr (SI == NS - 1) {
       const int t = thr(T::A, tid);
 #pragma unroll
       for (int k = 0; k < T::KB; ++k) store(t + k * TPT, v[k]);
     } else {
       cpx<C> w[St<SI + 1>::KB][St<SI + 1>::R];
       put<SI, 0>(lds, v, tid);
-      __syncthreads();
+      sync();
       get<SI + 1, 0>(lds, w, tid);
-      __syncthreads();
+      sync();
       put<SI, 1>(lds, v, tid);
-      __syncthreads();
+      sync();
       get<SI + 1, 1>(lds, w, tid);
-      if constexpr (SI + 1 < NS - 1) __syncthreads();  // the next exchange rewrites LDS
+      if constexpr (SI + 1 < NS - 1) sync();  // the next exchange rewrites LDS
       from<SI + 1>(w, lds, tw, tid, store);
     }
   }
 
   // load(b, m): element b + m * (N / R0) of this thread's input column.
-  // store(b, v): v[m] = element b + m * (N / RL) of its output column.
+  // store(b, v): v[m] = element b + m * (N / RL) of its output column, or
+  // store(v): all of them, v[k][m] for b = thr(AOUT, tid) + k * TPT.
   template <class Load, class Store>
   static __device__ __forceinline__ void run(C *lds, const cpx<C> *__restrict__ tw, int tid,
                                              Load &&load, Store &&store) {
@@ -139,6 +155,45 @@ struct TileEngine {
 #pragma unroll
       for (int m = 0; m < T::R; ++m) v[k][m] = load(t + k * TPT, m);
     from<0>(v, lds, tw, tid, store);
+  }
+};
+
+// The chain in reverse order.
+template <class Ch, class = std::make_integer_sequence<int, Ch::count>>
+struct ReversedChain;
+template <class Ch, int... I>
+struct ReversedChain<Ch, std::integer_sequence<int, I...>> {
+  using type = Chain<Ch::radix(Ch::count - 1 - I)...>;
+};
+
+// Two transforms of one length with a product in between (the convolutions of
+// kernels_conv.hpp and kernels_cz.hpp), W members of TPT threads. The last
+// stage of the first leaves a thread elements b + m * (N / RL), which are the
+// inputs of a first stage of radix RL: the second transform runs the chain in
+// reverse and takes them from registers. Against a transform through LDS in
+// natural order, a pass over LDS and the second transform's stage 0 this saves
+// one of 2 NS - 1 exchanges, and the split exchange half of the LDS.
+template <typename C, int W, int TPT, class Ch>
+struct ConvTile {
+  using First = TileEngine<C, W, TPT, Ch, false, false>;
+  using Second = TileEngine<C, W, TPT, typename ReversedChain<Ch>::type, false, false>;
+  static constexpr int N = Ch::N;
+  static constexpr int R = Ch::radix(Ch::count - 1);  // the radix on both sides of the product
+  static constexpr int NB = N / R, KB = NB / TPT;
+  static constexpr size_t LDS_BYTES =
+      First::LDS_BYTES > Second::LDS_BYTES ? First::LDS_BYTES : Second::LDS_BYTES;
+
+  // tw: the chain's twiddles, then those of the reversed chain. load(b, m) as
+  // TileEngine::run; mid(v): v[k][m] = element t + k TPT + m NB of the first
+  // transform, replaced by the second's input; store(b, v) as TileEngine::run.
+  template <class Load, class Mid, class Store>
+  static __device__ __forceinline__ void run(C *lds, const cpx<C> *__restrict__ tw, int tid,
+                                             Load &&load, Mid &&mid, Store &&store) {
+    First::run(lds, tw, tid, load, [&](cpx<C> (&v)[KB][R]) {
+      mid(v);
+      First::sync();  // the first's last reads are done
+      Second::template from<0>(v, lds, tw + Ch::tw_size(), tid, store);
+    });
   }
 };
 
