@@ -141,9 +141,9 @@ __global__ void __launch_bounds__(BLOCK) k_flex_c2r(FlexArgs f) {
         const int e = b + o;
         cpx<C> A = ST::ld(at_u32(X + (int64_t)o * is, gi + b * is));
         cpx<C> B = ST::ld(at_u32(X, gi + (m - e) * is));
-        const C s0 = e == 0 ? C(1) : hw, s1 = e == 0 ? C(0) : hw;
-        A = {s0 * A.x, s1 * A.y};
-        B = {s0 * B.x, s1 * B.y};
+        // X[0] and X[m] count as real, whatever their imaginary parts hold
+        A = {e == 0 ? A.x : hw * A.x, e == 0 ? C(0) : hw * A.y};
+        B = {e == 0 ? B.x : hw * B.x, e == 0 ? C(0) : hw * B.y};
         const cpx<C> s = {A.x + B.x, A.y - B.y};        // A + conj B
         const cpx<C> d = {A.x - B.x, A.y + B.y};        // A - conj B
         const cpx<C> wd = cconj_mul(d, at_u32(W + o, b));  // W^{-e} (A - conj B)

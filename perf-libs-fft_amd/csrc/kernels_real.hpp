@@ -35,6 +35,28 @@ __device__ __forceinline__ cpx<typename ST::C> load_pair(const typename ST::Rs *
 }
 
 // ---------------------------------------------------------------------------
+// Short packed members (at most 512 bytes): a thread's strided elements open a
+// line per few lanes. The block's members are consecutive: they are copied
+// through LDS with whole-line accesses on both sides. Bound by memory: R2C +
+// C2R of 2^24 reals as members of 64 in FP32 99 -> 68 us, FP64 68 -> 66 (half
+// as many); FP64 members of 128 (1 KB) are at 61 us without, 67 with.
+// ---------------------------------------------------------------------------
+template <class Eng>
+constexpr bool short_real() {
+  return Eng::NFIX > 0 && Eng::NFIX * sizeof(cpx<typename Eng::C>) <= 512;
+}
+
+// `rows` rows of N consecutive values at the LDS rows (element k of row r at
+// r * lper + lds_pad(k)), by T threads
+template <int N, int T, int PAD, class Move>
+__device__ __forceinline__ void short_rows(int rows, int lper, Move &&move) {
+  for (int i = threadIdx.x; i < rows * N; i += T) {
+    const int r = i / N, k = i % N;
+    move(r * lper + lds_pad<PAD>(k), i);
+  }
+}
+
+// ---------------------------------------------------------------------------
 // R2C, even n = 2m. flags bit0: reals may be read in pairs (unit stride,
 // even distance). aux0: W_n^k, k = 0..m/2 (forward sign).
 // ---------------------------------------------------------------------------
@@ -58,6 +80,39 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
   const cpx<C> *W = static_cast<const cpx<C> *>(a.aux0);
   // flags bit1: interior bins doubled (the adjoint of C2R)
   const C h = (a.flags & 2) ? C(1) : C(0.5);
+  if constexpr (short_real<Eng>()) {
+    constexpr int M = Eng::NFIX, T = TPT * TPB;
+    if (pair_ok && os == 1 && a.idist == 2 * M && a.odist == M + 1) {
+      const int rows = (int)(a.count - tr + g < TPB ? a.count - tr + g : TPB);
+      const int lper = Eng::lds_per(M);
+      cpx<C> *all = dyn_lds<C>();
+      const E *src = reinterpret_cast<const E *>(a.in) + (tr - g) * M;
+      E *dst = static_cast<E *>(a.out) + (tr - g) * (M + 1);
+      short_rows<M, T, Eng::PAD>(rows, lper, [&](int p, int i) { all[p] = ST::ld(src[i]); });
+      __syncthreads();
+      Eng::template run<true, true>(
+          a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, true,
+          [&](int) { return cpx<C>{C(0), C(0)}; }, [&](int, cpx<C>) {});
+      for (int k = t; 2 * k <= M; k += TPT) {
+        cpx<C> *zk = lds + lds_pad<Eng::PAD>(k), *zm = lds + lds_pad<Eng::PAD>(M - k);
+        if (k == 0) {
+          const cpx<C> z0 = *zk;
+          *zk = {z0.x + z0.y, C(0)};
+          *zm = {z0.x - z0.y, C(0)};  // slot M
+          continue;
+        }
+        const cpx<C> A = *zk, B = *zm;
+        const cpx<C> xe = {h * (A.x + B.x), h * (A.y - B.y)};
+        const cpx<C> xo = {h * (A.y + B.y), h * (B.x - A.x)};  // -i (A - conj B) / 2
+        const cpx<C> wx = cmul(W[k], xo);
+        *zk = cadd(xe, wx);
+        if (2 * k != M) *zm = {xe.x - wx.x, wx.y - xe.y};
+      }
+      __syncthreads();
+      short_rows<M + 1, T, Eng::PAD>(rows, lper, [&](int p, int i) { dst[i] = ST::st(all[p]); });
+      return;
+    }
+  }
   // output bins k and m-k from Z[k], Z[m-k]; so = output stride (1 when
   // known at compile time)
   auto post = [&](int k, cpx<C> w, int64_t so) {
@@ -168,7 +223,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even_split(KArgs a) {
   static_assert(2 * M == 2 * RL * NB, "n = 2 RL NB");
   cpx<C> z[KB * RL];
   EM::run_keep(lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-               [&](int e) { return load_pair<ST>(x, e, is, pair_ok); }, z);
+               in_bursts<8>([&](int e) { return load_pair<ST>(x, e, is, pair_ok); }), z);
   if (!valid) return;
   auto body = [&](auto unit) {
     constexpr bool U = decltype(unit)::value;  // unit output stride
@@ -358,6 +413,40 @@ __global__ void __launch_bounds__(Eng::TPT *TPB)
       y[(int64_t)(2 * e + 1) * os] = ST::str(v.y);
     }
   };
+  if constexpr (short_real<Eng>() && Eng::REGS_IN) {
+    constexpr int M = Eng::NFIX, T = TPT * TPB;
+    if (pair_ok && is == 1 && a.idist == M + 1 && a.odist == 2 * M) {
+      using Ch = typename Eng::Ch;
+      constexpr int R0 = Ch::radix(0), NB = M / R0, KB = (NB + TPT - 1) / TPT;
+      const int rows = (int)(a.count - tr + g < TPB ? a.count - tr + g : TPB);
+      const int lper = Eng::lds_per(M);
+      cpx<C> *all = dyn_lds<C>();
+      const E *src = static_cast<const E *>(a.in) + (tr - g) * (M + 1);
+      E *dst = reinterpret_cast<E *>(a.out) + (tr - g) * M;
+      short_rows<M + 1, T, Eng::PAD>(rows, lper, [&](int p, int i) { all[p] = ST::ld(src[i]); });
+      __syncthreads();
+      cpx<C> vin[KB * R0];
+#pragma unroll
+      for (int k = 0; k < KB; ++k)
+#pragma unroll
+        for (int j = 0; j < R0; ++j) {
+          int e = t + k * TPT;
+          if (NB % TPT != 0) e = e < NB ? e : NB - 1;
+          e += j * NB;
+          const cpx<C> A = lds[lds_pad<Eng::PAD>(e)], B = lds[lds_pad<Eng::PAD>(M - e)];
+          const C ax = e == 0 ? A.x : hw * A.x, ay = e == 0 ? C(0) : hw * A.y;
+          const C bx = e == 0 ? B.x : hw * B.x, by = e == 0 ? C(0) : hw * B.y;
+          const cpx<C> sm = {ax + bx, ay - by}, d = {ax - bx, ay + by};  // A +- conj B
+          const cpx<C> wd = cconj_mul(d, W[e]);
+          vin[k * R0 + j] = cswap(cpx<C>{sm.x - wd.y, sm.y + wd.x});
+        }
+      __syncthreads();  // the bins are read; the first exchange rewrites LDS
+      Eng::E::template run_regs<true>(vin, lds, static_cast<const cpx<C> *>(a.tw), t,
+                                      [&](int, cpx<C>) {}, true);
+      short_rows<M, T, Eng::PAD>(rows, lper, [&](int p, int i) { dst[i] = ST::st(cswap(all[p])); });
+      return;
+    }
+  }
   // Z'[e] for stage 0, w = W_n^e; si = input stride (1 when known at
   // compile time)
   auto pre = [&](int e, cpx<C> w, int64_t si) {
