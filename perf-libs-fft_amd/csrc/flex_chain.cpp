@@ -57,12 +57,14 @@ template <class F>
 int conflicts(int slots, F &&addr) {
   int worst = 0;
   for (int h = 0; h < 64; h += slots) {
-    int cnt[64] = {0};
-    std::set<int64_t> seen;
+    int cnt[32] = {0};
+    int64_t at[32][32];  // the distinct addresses of each slot
     for (int l = h; l < h + slots; ++l) {
       const int64_t a = addr(l);
-      if (!seen.insert(a).second) continue;  // same address: broadcast
-      worst = std::max(worst, ++cnt[a % slots]);
+      const int s = (int)(a % slots);
+      if (std::find(at[s], at[s] + cnt[s], a) != at[s] + cnt[s]) continue;  // broadcast
+      at[s][cnt[s]++] = a;
+      worst = std::max(worst, cnt[s]);
     }
   }
   return worst - 1;
@@ -164,6 +166,7 @@ bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int 
         bc = c;
         bp = p;
       }
+      if (c < 64) break;  // none: a larger pad cannot rank better
     }
     const int64_t GP = G + bp;
     d.st[s].wr_gp = (int)GP;

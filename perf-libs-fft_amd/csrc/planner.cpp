@@ -170,8 +170,8 @@ hipError_t EngineData::init(const Choice &c, int64_t len) {
     }
     std::vector<double> t = stockham_twiddles(c.chain);
     if (c.e->conv_lds) {
-      const std::vector<double> r =
-          stockham_twiddles(std::vector<int>(c.chain.rbegin(), c.chain.rend()));
+      const std::vector<int> rev(c.chain.rbegin(), c.chain.rend());
+      const std::vector<double> r = rev == c.chain ? t : stockham_twiddles(rev);
       t.insert(t.end(), r.begin(), r.end());
     }
     hipError_t err = upload_table(tw, t, c.e->prec);
