@@ -102,21 +102,32 @@ static hipError_t bluestein_kernel(int64_t n, int64_t M, const std::vector<doubl
   return dft_f64_gpu(*B, M, 1);
 }
 
+// [j][i], j < rows, i < count: W_M^{j step i}; transposed: [i][j]
+static void cz_table(std::vector<double> *t, int64_t M, int64_t rows, int64_t count,
+                     int64_t step, bool transposed) {
+  const int64_t no = transposed ? count : rows, ni = transposed ? rows : count;
+  for (int64_t o = 0; o < no; ++o)
+    for (int64_t i = 0; i < ni; ++i) {
+      double re, im;
+      unit_root(o * i * step % M, M, &re, &im);
+      t->push_back(re);
+      t->push_back(-im);
+    }
+}
+
 std::vector<double> cz_mid_twiddles(int64_t n1, const Choice &mid) {
   const int64_t n2 = mid.e->n, R = mid.chain[0], NB = n2 / R, M = n1 * n2;
   std::vector<double> t;
-  t.reserve(2 * (size_t)(n1 * (NB + R)));
-  auto table = [&](int64_t count, int64_t step) {  // W_M^{k1 step i}, i < count
-    for (int64_t k1 = 0; k1 < n1; ++k1)
-      for (int64_t i = 0; i < count; ++i) {
-        double re, im;
-        unit_root(k1 * step * i % M, M, &re, &im);
-        t.push_back(re);
-        t.push_back(-im);
-      }
-  };
-  table(NB, 1);
-  table(R, NB);
+  cz_table(&t, M, n1, NB, 1, false);
+  cz_table(&t, M, n1, R, NB, false);
+  return t;
+}
+
+std::vector<double> cz_col_twiddles(const Choice &col, int64_t n2) {
+  const int64_t n1 = col.e->n, R = col.chain.back(), NB = n1 / R, M = n1 * n2;
+  std::vector<double> t;
+  cz_table(&t, M, n2, NB, 1, true);
+  cz_table(&t, M, n2, R, NB, true);
   return t;
 }
 
@@ -290,25 +301,7 @@ class ChirpZ3Node : public Node {
     if (err == hipSuccess) err = eout_.init(cout_, n1_);
     if (err != hipSuccess) return err;
     const int64_t M = n1_ * n2_;
-    int lg = 0;
-    while ((int64_t(1) << lg) < M) ++lg;
-    shift_ = (lg + 1) / 2;
-    const int64_t nlo = int64_t(1) << shift_, nhi = ((M - 1) >> shift_) + 1;
-    // W_M split table: lo[r] = W_M^r (r < 2^shift), then hi[q] = W_M^{q 2^shift}
-    std::vector<double> sp;
-    for (int64_t r = 0; r < nlo; ++r) {
-      double re, im;
-      unit_root(r, M, &re, &im);
-      sp.push_back(re);
-      sp.push_back(-im);
-    }
-    for (int64_t q = 0; q < nhi; ++q) {
-      double re, im;
-      unit_root(q * nlo, M, &re, &im);
-      sp.push_back(re);
-      sp.push_back(-im);
-    }
-    err = upload_table(split_, sp, prec_);
+    err = upload_table(tcol_, cz_col_twiddles(cin_, n2_), prec_);
     if (err == hipSuccess) err = upload_table(tmid_, cz_mid_twiddles(n1_, cmid_), prec_);
     if (err != hipSuccess) return err;
     std::vector<double> c = chirp_table(n_), B;
@@ -343,11 +336,10 @@ class ChirpZ3Node : public Node {
     for (int64_t b0 = 0; b0 < batch_; b0 += chunk) {
       const int64_t cb = std::min(chunk, batch_ - b0);
       KArgs a{};
-      a.aux0 = split_.p;
+      a.aux0 = tcol_.p;
       a.n1 = n1_;
       a.n2 = n2_;
       a.bigdist = n_;
-      a.shift = shift_;
       // 1. chirp-in columns
       a.in = static_cast<const char *>(in) + (size_t)(b0 * id_) * eb;
       a.out = work;
@@ -358,8 +350,7 @@ class ChirpZ3Node : public Node {
       a.aux1 = c_.p;
       a.n = n1_;
       a.count = cb * n2_;
-      hipError_t err = cin_.e->launch(a, (a.count + cin_.e->tpb - 1) / cin_.e->tpb,
-                                      cin_.e->lds_bytes(n1_), s);
+      hipError_t err = cin_.e->launch(a, a.count / cin_.e->tpb, cin_.e->lds_bytes(n1_), s);
       // 2. rows: DFT_n2, x B, the inverse's first DFT_n2
       if (err == hipSuccess) {
         a.tw = emid_.tw.p;
@@ -380,7 +371,7 @@ class ChirpZ3Node : public Node {
         a.aux1 = c_.p;
         a.n = n1_;
         a.count = cb * n2_;
-        err = cout_.e->launch(a, (a.count + cout_.e->tpb - 1) / cout_.e->tpb,
+        err = cout_.e->launch(a, a.count / cout_.e->tpb,
                               cout_.e->lds_bytes(n1_), s);
       }
       if (err != hipSuccess) return err;
@@ -402,8 +393,7 @@ class ChirpZ3Node : public Node {
   int64_t batch_, is_, id_, os_, od_, chunk_;
   Choice cin_, cmid_, cout_;
   EngineData ein_, emid_, eout_;
-  int shift_ = 0;
-  DevMem split_, tmid_, B_, c_;
+  DevMem tcol_, tmid_, B_, c_;
 };
 
 // Rader for a prime n in three passes over N = n - 1 = n1 * n2
@@ -425,25 +415,7 @@ class Rader3Node : public Node {
     if (err == hipSuccess) err = eout_.init(cout_, n1_);
     if (err != hipSuccess) return err;
     const int64_t N = n1_ * n2_;
-    int lg = 0;
-    while ((int64_t(1) << lg) < N) ++lg;
-    shift_ = (lg + 1) / 2;
-    const int64_t nlo = int64_t(1) << shift_, nhi = ((N - 1) >> shift_) + 1;
-    // W_N split table: lo[r] = W_N^r (r < 2^shift), then hi[q] = W_N^{q 2^shift}
-    std::vector<double> sp;
-    for (int64_t r = 0; r < nlo; ++r) {
-      double re, im;
-      unit_root(r, N, &re, &im);
-      sp.push_back(re);
-      sp.push_back(-im);
-    }
-    for (int64_t q = 0; q < nhi; ++q) {
-      double re, im;
-      unit_root(q * nlo, N, &re, &im);
-      sp.push_back(re);
-      sp.push_back(-im);
-    }
-    err = upload_table(split_, sp, prec_);
+    err = upload_table(tcol_, cz_col_twiddles(cin_, n2_), prec_);
     if (err == hipSuccess) err = upload_table(tmid_, cz_mid_twiddles(n1_, cmid_), prec_);
     if (err != hipSuccess) return err;
     gen_ = group_generator(n_);
@@ -493,12 +465,11 @@ class Rader3Node : public Node {
     for (int64_t b0 = 0; b0 < batch_; b0 += chunk) {
       const int64_t nb = std::min(chunk, batch_ - b0);
       KArgs a{};
-      a.aux0 = split_.p;
+      a.aux0 = tcol_.p;
       a.aux1 = perm_.p;
       a.aux3 = slots;
       a.n1 = n1_;
       a.n2 = n2_;
-      a.shift = shift_;
       // 1. permuted-input columns
       a.in = static_cast<const char *>(in) + (size_t)(b0 * id_) * eb;
       a.out = work;
@@ -508,8 +479,7 @@ class Rader3Node : public Node {
       a.desc = ein_.d();
       a.n = n1_;
       a.count = nb * n2_;
-      hipError_t err = cin_.e->launch(a, (a.count + cin_.e->tpb - 1) / cin_.e->tpb,
-                                      cin_.e->lds_bytes(n1_), s);
+      hipError_t err = cin_.e->launch(a, a.count / cin_.e->tpb, cin_.e->lds_bytes(n1_), s);
       // 2. rows: DFT_n2, x B, the inverse's first DFT_n2 (A_0 kept)
       if (err == hipSuccess) {
         a.in = nullptr;
@@ -534,7 +504,7 @@ class Rader3Node : public Node {
         a.aux1 = perm_.p;
         a.n = n1_;
         a.count = nb * n2_;
-        err = cout_.e->launch(a, (a.count + cout_.e->tpb - 1) / cout_.e->tpb,
+        err = cout_.e->launch(a, a.count / cout_.e->tpb,
                               std::max<size_t>(81 * 1024, cout_.e->lds_bytes(n1_)), s);
       }
       if (err != hipSuccess) return err;
@@ -556,9 +526,8 @@ class Rader3Node : public Node {
   int64_t batch_, is_, id_, os_, od_, chunk_;
   Choice cin_, cmid_, cout_;
   EngineData ein_, emid_, eout_;
-  int shift_ = 0;
   int64_t gen_ = 0;
-  DevMem split_, tmid_, B_, perm_;
+  DevMem tcol_, tmid_, B_, perm_;
 };
 
 // The most balanced split N = n1 * n2 (n1 a power of two) with compiled
@@ -572,7 +541,8 @@ static bool rd3_choice(int64_t N, int prec, bool bwd, int64_t *n1_out, Choice *c
     Choice ci = choose(KK_RD_COL_IN, n1, prec, bwd);
     Choice cm = choose(KK_CZ_ROW_MID, n2, prec, bwd);
     Choice co = choose(KK_RD_COL_OUT, n1, prec, bwd);
-    if (!ci.e || !cm.e || !co.e || n1 % cm.e->tpb) continue;
+    if (!ci.e || !cm.e || !co.e || n1 % cm.e->tpb || n2 % ci.e->tpb || n2 % co.e->tpb)
+        continue;
     const double bal = std::fabs(std::log((double)n1 / (double)n2));
     if (bal < best) {
       best = bal;
@@ -602,7 +572,8 @@ bool cz3_choice(int64_t n, int prec, bool bwd, Cz3Choice *out) {
       Choice ci = choose(KK_CZ_COL_IN, n1, prec, bwd);
       Choice cm = choose(KK_CZ_ROW_MID, n2, prec, bwd);
       Choice co = choose(KK_CZ_COL_OUT, n1, prec, bwd);
-      if (!ci.e || !cm.e || !co.e || n1 % cm.e->tpb) continue;
+      if (!ci.e || !cm.e || !co.e || n1 % cm.e->tpb || n2 % ci.e->tpb || n2 % co.e->tpb)
+        continue;
       out->M = M;
       out->n1 = n1;
       out->cin = ci;

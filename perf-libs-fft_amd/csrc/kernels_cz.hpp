@@ -16,11 +16,10 @@
 //      times c_m, stored for m < n.
 // The backward transform is swap o forward o swap on the input and output.
 //
-// KArgs of all three: tw = the engine's Stockham twiddles, aux0 = W_M split
-// table (lo: 2^shift entries, then hi), n = engine length, n1, n2 = the
-// sides, bigdist = the transform length n, count = columns (members * n2) or
+// KArgs of all three: tw = the engine's Stockham twiddles, n = engine length,
+// n1, n2 = the sides, bigdist = the transform length n, count = columns (members * n2) or
 // rows (members * n1). Pass 1: in = input (storage type, istride, idist),
-// out = workspace, aux1 = chirp. Pass 2: out = workspace, aux0 = its own
+// out = workspace, aux0 = its twiddles (CzTile::put), aux1 = chirp. Pass 2: out = workspace, aux0 = its own
 // twiddles (k_cz_row_mid), aux1 = B. Pass 3:
 // in = workspace, out = output (ostride, odist), aux1 = chirp.
 // Gathered launch (aux2 = CzMember records, one per member of the launch;
@@ -33,45 +32,69 @@
 
 namespace plf {
 
-template <typename C>
-__device__ __forceinline__ cpx<C> cz_twiddle(const cpx<C> *__restrict__ split, int shift,
-                                             int64_t e) {
-  const cpx<C> *hi = split + (int64_t(1) << shift);
-  return cmul(hi[e >> shift], split[e & ((int64_t(1) << shift) - 1)]);
-}
+// A block's tile of a column pass: W neighbouring columns c of one member
+// (n2 % W == 0), lanes along the columns, on the split exchange. The chirp-z
+// passes are bound by memory, Rader's by their 8-byte gathers and scatters
+// (a line each). 512 members of 65537: in 270 -> 236 us, out 267 -> 255 us
+// against the full exchange with a split twiddle table; 800 members of 20011,
+// all three passes, 472 -> 420 us.
+template <typename C, int W, int TPT, class Ch>
+struct CzTile {
+  using T = TileEngine<C, W, TPT, Ch, true, true>;
+  static constexpr int R0 = Ch::radix(0), NB0 = Ch::N / R0;
+  static constexpr int RL = Ch::radix(Ch::count - 1), NBL = Ch::N / RL;
+  uint32_t n2, bi, c;
+  int t;
+  __device__ __forceinline__ explicit CzTile(const KArgs &a) {
+    n2 = (uint32_t)a.n2;
+    const uint32_t tpm = n2 / W, bx = (uint32_t)xcd_block(blockIdx.x, gridDim.x);
+    bi = bx / tpm;
+    c = (bx % tpm) * W + threadIdx.x % W;
+    t = threadIdx.x / W;
+  }
+  // outputs b + m NBL of the column, twiddled by W_M^{c k1}, to the workspace;
+  // T1[b][c] and T2[m][c] are read along the columns (the split table of the
+  // other exponents took two gathers an element)
+  __device__ __forceinline__ void put(const KArgs &a, cpx<C> *ws, int b,
+                                      const cpx<C> (&v)[RL]) const {
+    const cpx<C> *t1 = static_cast<const cpx<C> *>(a.aux0);
+    const cpx<C> *t2 = t1 + (uint32_t)NBL * n2;
+    const cpx<C> wb = at_u32(t1, (uint32_t)b * n2 + c);
+    cpx<C> y[RL];
+#pragma unroll
+    for (int m = 0; m < RL; ++m)
+      y[m] = cmul(v[m], m == 0 ? wb : cmul(wb, at_u32(t2, (uint32_t)m * n2 + c)));
+#pragma unroll
+    for (int m = 0; m < RL; ++m) ws[(uint32_t)(b + m * NBL) * n2 + c] = y[m];
+  }
+};
 
-template <typename S, bool BWD, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_col_in(KArgs a) {
+template <typename S, bool BWD, int W, int TPT, class Ch>
+__global__ void __launch_bounds__(W *TPT) k_cz_col_in(KArgs a) {
   using ST = StorageT<S>;
   using E = typename ST::E;
-  using C = typename Eng::C;
-  const int g = threadIdx.x % TPB;
-  const int t = threadIdx.x / TPB;
-  const int64_t col = xcd_block(blockIdx.x, gridDim.x) * TPB + g;
-  const bool valid = col < a.count;
-  const int64_t n1 = a.n1, n2 = a.n2;
-  const int64_t bi = valid ? col / n2 : 0, c2 = valid ? col % n2 : 0;
+  using C = typename ST::C;
+  using Z = CzTile<C, W, TPT, Ch>;
+  const Z z(a);
   const CzMember *mt = static_cast<const CzMember *>(a.aux2);
-  const int64_t nn = mt ? mt[bi].n : a.bigdist;
-  const E *in = static_cast<const E *>(a.in) + (mt ? mt[bi].in_off : bi * a.idist);
-  cpx<C> *ws = static_cast<cpx<C> *>(a.out) + (mt ? mt[bi].ws_off : bi * n1 * n2) + c2;
-  const cpx<C> *split = static_cast<const cpx<C> *>(a.aux0);
-  const cpx<C> *chirp = static_cast<const cpx<C> *>(a.aux1) + (mt ? mt[bi].chirp_off : 0);
+  const uint32_t nn = (uint32_t)(mt ? mt[z.bi].n : a.bigdist);
+  const E *in = static_cast<const E *>(a.in) + (mt ? mt[z.bi].in_off : z.bi * a.idist);
+  cpx<C> *ws = static_cast<cpx<C> *>(a.out) +
+               (mt ? mt[z.bi].ws_off : (int64_t)z.bi * Ch::N * z.n2);
+  const cpx<C> *chirp = static_cast<const cpx<C> *>(a.aux1) + (mt ? mt[z.bi].chirp_off : 0);
   const int64_t is = mt ? 1 : a.istride;
-  const int shift = a.shift;
-  cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  Eng::template run<false>(
-      a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int b, int o) {
-        // zero padding: skipped where it is all padding (the same for every
-        // thread), otherwise selected after a load of element 0
-        if (n2 * o >= nn) return cpx<C>{C(0), C(0)};
-        const int64_t j0 = c2 + n2 * (b + o), j = j0 < nn ? j0 : 0;
+  Z::T::run(
+      reinterpret_cast<C *>(dyn_lds<C>()), static_cast<const cpx<C> *>(a.tw), threadIdx.x,
+      [&](int b, int m) {
+        // n <= M / 2 + 1, as M >= 2n - 2: the upper half is padding; below it
+        // padding is selected after a load of element 0
+        if (2 * m * Z::NB0 > Ch::N) return cpx<C>{C(0), C(0)};
+        const uint32_t j0 = z.c + z.n2 * (uint32_t)(b + m * Z::NB0), j = j0 < nn ? j0 : 0;
         cpx<C> v = ST::ld(in[j * is]);
         v = cmul(BWD ? cswap(v) : v, chirp[j]);
         return cpx<C>{j0 < nn ? v.x : C(0), j0 < nn ? v.y : C(0)};
       },
-      [&](int k1, cpx<C> v) { ws[(int64_t)k1 * n2] = cmul(v, cz_twiddle(split, shift, c2 * k1)); });
+      [&](int b, const cpx<C> (&v)[Z::RL]) { z.put(a, ws, b, v); });
 }
 
 // Row pass, on the two-transform tile engine (ConvTile): W rows of TPT threads
@@ -117,32 +140,32 @@ __global__ void __launch_bounds__(TPT *W) k_cz_row_mid(KArgs a) {
       });
 }
 
-template <typename S, bool BWD, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_col_out(KArgs a) {
+template <typename S, bool BWD, int W, int TPT, class Ch>
+__global__ void __launch_bounds__(W *TPT) k_cz_col_out(KArgs a) {
   using ST = StorageT<S>;
   using E = typename ST::E;
-  using C = typename Eng::C;
-  const int g = threadIdx.x % TPB;
-  const int t = threadIdx.x / TPB;
-  const int64_t col = xcd_block(blockIdx.x, gridDim.x) * TPB + g;
-  const bool valid = col < a.count;
-  const int64_t n1 = a.n1, n2 = a.n2;
-  const int64_t bi = valid ? col / n2 : 0, c2 = valid ? col % n2 : 0;
+  using C = typename ST::C;
+  using Z = CzTile<C, W, TPT, Ch>;
+  const Z z(a);
   const CzMember *mt = static_cast<const CzMember *>(a.aux2);
-  const int64_t nn = mt ? mt[bi].n : a.bigdist;
-  const cpx<C> *ws = static_cast<const cpx<C> *>(a.in) + (mt ? mt[bi].ws_off : bi * n1 * n2) + c2;
-  E *out = static_cast<E *>(a.out) + (mt ? mt[bi].out_off : bi * a.odist);
-  const cpx<C> *chirp = static_cast<const cpx<C> *>(a.aux1) + (mt ? mt[bi].chirp_off : 0);
+  const uint32_t nn = (uint32_t)(mt ? mt[z.bi].n : a.bigdist);
+  const cpx<C> *ws = static_cast<const cpx<C> *>(a.in) +
+                     (mt ? mt[z.bi].ws_off : (int64_t)z.bi * Ch::N * z.n2);
+  E *out = static_cast<E *>(a.out) + (mt ? mt[z.bi].out_off : z.bi * a.odist);
+  const cpx<C> *chirp = static_cast<const cpx<C> *>(a.aux1) + (mt ? mt[z.bi].chirp_off : 0);
   const int64_t os = mt ? 1 : a.ostride;
-  cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  Eng::template run<false>(
-      a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) { return ws[(int64_t)e * n2]; },
-      [&](int m1, cpx<C> v) {
-        const int64_t m = c2 + n2 * m1;
-        if (m < nn) {
-          const cpx<C> y = cmul(cswap(v), chirp[m]);
-          out[m * os] = ST::st(BWD ? cswap(y) : y);
+  Z::T::run(
+      reinterpret_cast<C *>(dyn_lds<C>()), static_cast<const cpx<C> *>(a.tw), threadIdx.x,
+      [&](int b, int m) { return ws[(uint32_t)(b + m * Z::NB0) * z.n2 + z.c]; },
+      [&](int b, const cpx<C> (&v)[Z::RL]) {
+#pragma unroll
+        for (int m = 0; m < Z::RL; ++m) {
+          if (2 * m * Z::NBL > Ch::N) continue;  // n <= M / 2 + 1
+          const uint32_t j = z.c + z.n2 * (uint32_t)(b + m * Z::NBL);
+          if (j < nn) {
+            const cpx<C> y = cmul(cswap(v[m]), chirp[j]);
+            out[j * os] = ST::st(BWD ? cswap(y) : y);
+          }
         }
       });
 }
@@ -156,63 +179,60 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_cz_col_out(KArgs a) {
 // KArgs as for the chirp-z passes, except: aux1 = perm (int32, N entries)
 // in the column passes, aux3 = two slots per member of the launch (x_0,
 // A_0; compute precision) and bigdist unused (no padding).
-template <typename S, bool BWD, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_rd_col_in(KArgs a) {
+template <typename S, bool BWD, int W, int TPT, class Ch>
+__global__ void __launch_bounds__(W *TPT) k_rd_col_in(KArgs a) {
   using ST = StorageT<S>;
   using E = typename ST::E;
-  using C = typename Eng::C;
-  const int g = threadIdx.x % TPB;
-  const int t = threadIdx.x / TPB;
-  const int64_t col = xcd_block(blockIdx.x, gridDim.x) * TPB + g;
-  const bool valid = col < a.count;
-  const int64_t n1 = a.n1, n2 = a.n2;
-  const int64_t bi = valid ? col / n2 : 0, c2 = valid ? col % n2 : 0;
-  const E *in = static_cast<const E *>(a.in) + bi * a.idist;
-  cpx<C> *ws = static_cast<cpx<C> *>(a.out) + bi * n1 * n2 + c2;
-  const cpx<C> *split = static_cast<const cpx<C> *>(a.aux0);
-  const int *perm = static_cast<const int *>(a.aux1) + c2;
+  using C = typename ST::C;
+  using Z = CzTile<C, W, TPT, Ch>;
+  const Z z(a);
+  const E *in = static_cast<const E *>(a.in) + z.bi * a.idist;
+  cpx<C> *ws = static_cast<cpx<C> *>(a.out) + (int64_t)z.bi * Ch::N * z.n2;
+  const int *perm = static_cast<const int *>(a.aux1);
   const int64_t is = a.istride;
-  const int shift = a.shift;
-  if (valid && c2 == 0 && t == 0) {
+  if (z.c == 0 && z.t == 0) {
     const cpx<C> x0 = ST::ld(in[0]);
-    static_cast<cpx<C> *>(a.aux3)[2 * bi] = BWD ? cswap(x0) : x0;
+    static_cast<cpx<C> *>(a.aux3)[2 * z.bi] = BWD ? cswap(x0) : x0;
   }
-  cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  Eng::template run<false>(
-      a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) {
-        const cpx<C> v = ST::ld(in[(int64_t)perm[n2 * e] * is]);
+  Z::T::run(
+      reinterpret_cast<C *>(dyn_lds<C>()), static_cast<const cpx<C> *>(a.tw), threadIdx.x,
+      [&](int b, int m) {
+        const cpx<C> v = ST::ld(in[perm[z.n2 * (uint32_t)(b + m * Z::NB0) + z.c] * is]);
         return BWD ? cswap(v) : v;
       },
-      [&](int k1, cpx<C> v) { ws[(int64_t)k1 * n2] = cmul(v, cz_twiddle(split, shift, c2 * k1)); });
+      [&](int b, const cpx<C> (&v)[Z::RL]) { z.put(a, ws, b, v); });
 }
 
-template <typename S, bool BWD, int TPB, class Eng>
-__global__ void __launch_bounds__(Eng::TPT *TPB) k_rd_col_out(KArgs a) {
+template <typename S, bool BWD, int W, int TPT, class Ch>
+__global__ void __launch_bounds__(W *TPT) k_rd_col_out(KArgs a) {
   using ST = StorageT<S>;
   using E = typename ST::E;
-  using C = typename Eng::C;
-  const int g = threadIdx.x % TPB;
-  const int t = threadIdx.x / TPB;
-  const int64_t col = xcd_block(blockIdx.x, gridDim.x) * TPB + g;
-  const bool valid = col < a.count;
-  const int64_t n1 = a.n1, n2 = a.n2, N = n1 * n2;
-  const int64_t bi = valid ? col / n2 : 0, c2 = valid ? col % n2 : 0;
-  const cpx<C> *ws = static_cast<const cpx<C> *>(a.in) + bi * N + c2;
-  E *out = static_cast<E *>(a.out) + bi * a.odist;
+  using C = typename ST::C;
+  using Z = CzTile<C, W, TPT, Ch>;
+  const Z z(a);
+  const uint32_t N = Ch::N * z.n2;
+  const cpx<C> *ws = static_cast<const cpx<C> *>(a.in) + (int64_t)z.bi * N;
+  E *out = static_cast<E *>(a.out) + z.bi * a.odist;
   const int *perm = static_cast<const int *>(a.aux1);
-  const cpx<C> *slot = static_cast<const cpx<C> *>(a.aux3) + 2 * bi;
+  const cpx<C> *slot = static_cast<const cpx<C> *>(a.aux3) + 2 * z.bi;
   const cpx<C> x0 = slot[0];
   const int64_t os = a.ostride;
-  cpx<C> *lds = dyn_lds<C>() + g * Eng::lds_per(a.n);
-  Eng::template run<false>(
-      a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
-      [&](int e) { return ws[(int64_t)e * n2]; },
-      [&](int m1, cpx<C> v) {
-        const int64_t q = c2 + n2 * m1;
-        const cpx<C> r = cadd(x0, cswap(v));
-        out[(int64_t)perm[q == 0 ? 0 : N - q] * os] = ST::st(BWD ? cswap(r) : r);
-        if (q == 0) {
+  Z::T::run(
+      reinterpret_cast<C *>(dyn_lds<C>()), static_cast<const cpx<C> *>(a.tw), threadIdx.x,
+      [&](int b, int m) { return ws[(uint32_t)(b + m * Z::NB0) * z.n2 + z.c]; },
+      [&](int b, const cpx<C> (&v)[Z::RL]) {
+        int64_t at[Z::RL];
+#pragma unroll
+        for (int m = 0; m < Z::RL; ++m) {
+          const uint32_t q = z.c + z.n2 * (uint32_t)(b + m * Z::NBL);
+          at[m] = perm[q == 0 ? 0 : N - q] * os;
+        }
+#pragma unroll
+        for (int m = 0; m < Z::RL; ++m) {
+          const cpx<C> r = cadd(x0, cswap(v[m]));
+          out[at[m]] = ST::st(BWD ? cswap(r) : r);
+        }
+        if (z.c == 0 && b == 0) {
           const cpx<C> y0 = cadd(x0, slot[1]);
           out[0] = ST::st(BWD ? cswap(y0) : y0);
         }

@@ -211,9 +211,11 @@ inline void add_entry(std::vector<KEntry> &r, int kind, int prec, int n,
 // pass of the three-pass convolutions is one kernel for all storage types of a
 // compute type and both directions.
 #define PLF_CONV_LDS(S, TPT, TPB, ...)                                                     \
-  for (int i_ = 1; i_ <= 2; ++i_)                                                          \
-  r[r.size() - i_].conv_lds = ::plf::ConvTile<typename ::plf::StorageT<S>::C, TPB, TPT,     \
-                                              ::plf::Chain<__VA_ARGS__>>::LDS_BYTES
+  for (int i_ = 1; i_ <= 2; ++i_) {                                                        \
+    r[r.size() - i_].tile_lds = ::plf::ConvTile<typename ::plf::StorageT<S>::C, TPB, TPT,   \
+                                                ::plf::Chain<__VA_ARGS__>>::LDS_BYTES;     \
+    r[r.size() - i_].both_chains = true;                                                   \
+  }
 #define PLF_BLUE_TILE(S, PREC, TPT, TPB, ...)                                              \
   do {                                                                                     \
     using ChT = ::plf::Chain<__VA_ARGS__>;                                                 \
@@ -231,3 +233,19 @@ inline void add_entry(std::vector<KEntry> &r, int kind, int prec, int n,
                      run, run);                                                            \
     PLF_CONV_LDS(S, TPT, TPB, __VA_ARGS__);                                                \
   } while (0)
+// The column passes of the three-pass convolutions: K<S, BWD, W, TPT, Chain>.
+#define PLF_CZ_COL(K, KK, S, PREC, TPT, W, ...)                                            \
+  do {                                                                                     \
+    using ChT = ::plf::Chain<__VA_ARGS__>;                                                 \
+    ::plf::add_entry(r, ::plf::KK, PREC, ChT::N, {__VA_ARGS__}, TPT, W, 0, true,           \
+                     &::plf::launch_k<&::plf::K<S, false, W, TPT, ChT>, TPT * W>,          \
+                     &::plf::launch_k<&::plf::K<S, true, W, TPT, ChT>, TPT * W>);          \
+    for (int i_ = 1; i_ <= 2; ++i_)                                                        \
+      r[r.size() - i_].tile_lds = ::plf::TileEngine<typename ::plf::StorageT<S>::C, W, TPT, \
+                                                    ChT, true, true>::LDS_BYTES;           \
+  } while (0)
+#define PLF_CZ_COLS(S, PREC, TPT, W, ...)                                                  \
+  PLF_CZ_COL(k_cz_col_in, KK_CZ_COL_IN, S, PREC, TPT, W, __VA_ARGS__);                     \
+  PLF_CZ_COL(k_cz_col_out, KK_CZ_COL_OUT, S, PREC, TPT, W, __VA_ARGS__);                   \
+  PLF_CZ_COL(k_rd_col_in, KK_RD_COL_IN, S, PREC, TPT, W, __VA_ARGS__);                     \
+  PLF_CZ_COL(k_rd_col_out, KK_RD_COL_OUT, S, PREC, TPT, W, __VA_ARGS__)

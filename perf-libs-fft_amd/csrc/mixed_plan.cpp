@@ -499,11 +499,9 @@ std::unique_ptr<MixedPlan> MixedPlan::build(int prec, int fixed_bits, int dir, i
       m.ws_off = ws;
       ws += M;
     }
-    const auto spl = get_split(M);
-    g->split_off = spl.first;
-    g->shift = spl.second;
     hipError_t err = g->ein.init(g->cin, g->n1);
     if (err == hipSuccess) err = g->emid.init(g->cmid, g->n2);
+    if (err == hipSuccess) err = upload_table(g->tcol, cz_col_twiddles(g->cin, g->n2), prec);
     if (err == hipSuccess) err = upload_table(g->tmid, cz_mid_twiddles(g->n1, g->cmid), prec);
     if (err == hipSuccess) err = g->eout.init(g->cout, g->n1);
     if (err == hipSuccess)
@@ -624,14 +622,12 @@ hipError_t MixedPlan::enqueue(const void *in, void *out, void *ws, hipStream_t s
                                           g->c.e->lds_bytes(g->M), s);
     if (err != hipSuccess) return err;
   }
-  const size_t cb = 2 * (size_t)prec_compute_bytes(prec_);
   for (const auto &g : cz_groups_) {
     KArgs k{};
-    k.aux0 = static_cast<const char *>(aux_.p) + (size_t)g->split_off * cb;
+    k.aux0 = g->tcol.p;
     k.aux2 = g->members.p;
     k.n1 = g->n1;
     k.n2 = g->n2;
-    k.shift = g->shift;
     // 1. chirp-in columns
     k.in = in;
     k.out = ws;
@@ -639,8 +635,7 @@ hipError_t MixedPlan::enqueue(const void *in, void *out, void *ws, hipStream_t s
     k.tw = g->ein.tw.p;
     k.n = g->n1;
     k.count = g->count * g->n2;
-    hipError_t err = g->cin.e->launch(k, (k.count + g->cin.e->tpb - 1) / g->cin.e->tpb,
-                                      g->cin.e->lds_bytes(g->n1), s);
+    hipError_t err = g->cin.e->launch(k, k.count / g->cin.e->tpb, g->cin.e->lds_bytes(g->n1), s);
     // 2. rows (B tables in aux at the members' B offsets)
     if (err == hipSuccess) {
       k.tw = g->emid.tw.p;
@@ -656,8 +651,7 @@ hipError_t MixedPlan::enqueue(const void *in, void *out, void *ws, hipStream_t s
       k.tw = g->eout.tw.p;
       k.n = g->n1;
       k.count = g->count * g->n2;
-      err = g->cout.e->launch(k, (k.count + g->cout.e->tpb - 1) / g->cout.e->tpb,
-                              g->cout.e->lds_bytes(g->n1), s);
+      err = g->cout.e->launch(k, k.count / g->cout.e->tpb, g->cout.e->lds_bytes(g->n1), s);
     }
     if (err != hipSuccess) return err;
   }

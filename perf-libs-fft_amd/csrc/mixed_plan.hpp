@@ -52,9 +52,8 @@ class MixedPlan {
   struct CzGroup {
     Choice cin, cmid, cout;
     EngineData ein, emid, eout;
-    int64_t n1 = 0, n2 = 0, count = 0, split_off = 0;
-    int shift = 0;
-    DevMem tmid;     // the middle pass's twiddles
+    int64_t n1 = 0, n2 = 0, count = 0;
+    DevMem tcol, tmid;  // twiddles of the first and the middle pass
     DevMem members;  // CzMember records
   };
   std::vector<std::unique_ptr<CzGroup>> cz_groups_;

@@ -159,6 +159,8 @@ struct Cz3Choice {
 };
 // The middle pass's twiddles (k_cz_row_mid: T1, then T2) for n1 rows.
 std::vector<double> cz_mid_twiddles(int64_t n1, const Choice &mid);
+// The first pass's twiddles (CzTile::put: T1, then T2) for n2 columns.
+std::vector<double> cz_col_twiddles(const Choice &col, int64_t n2);
 bool cz3_choice(int64_t n, int prec, bool bwd, Cz3Choice *out);
 
 // Twiddle table of a Stockham radix chain, FORWARD sign, FP64:

@@ -169,7 +169,7 @@ hipError_t EngineData::init(const Choice &c, int64_t len) {
       return tw.upload(t.data(), t.size() * sizeof(uint16_t));
     }
     std::vector<double> t = stockham_twiddles(c.chain);
-    if (c.e->conv_lds) {
+    if (c.e->both_chains) {
       const std::vector<int> rev(c.chain.rbegin(), c.chain.rend());
       const std::vector<double> r = rev == c.chain ? t : stockham_twiddles(rev);
       t.insert(t.end(), r.begin(), r.end());

@@ -73,15 +73,15 @@ struct KEntry {
   bool xlane = false;   // cross-lane kernel: packed members only, lane twiddle table
   bool mfma = false;    // first stage on the matrix cores
   bool packed = false;  // members contiguous at distance n only
-  size_t conv_lds = 0;  // > 0: two-transform tile kernel (tw: the chain's twiddles, then those
-                        // of the reversed chain) of this many bytes of LDS
+  size_t tile_lds = 0;  // > 0: kernel on the tile engine with this many bytes of LDS
+  bool both_chains = false;  // tw: the chain's twiddles, then those of the reversed chain
   bool staged = false;  // one member per thread, global access staged through LDS
   KLaunch launch;
   std::string name() const;
   // LDS bytes of one block for engine length len
   size_t lds_bytes(int64_t len) const {
     if (!uses_lds) return 0;
-    if (conv_lds) return conv_lds;
+    if (tile_lds) return tile_lds;
     return (size_t)tpb * (size_t)(len + (len >> pad) + 1) * lds_scalars * prec_compute_bytes(prec);
   }
   // can the dynamic engine run this radix chain within pts points/thread
