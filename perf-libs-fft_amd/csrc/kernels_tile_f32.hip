@@ -15,13 +15,13 @@ void register_tiles_f32(std::vector<TileEntry> &r) {
   add_tile_c2c<S, 32, 16, 4, 16, 32>(r, P);
   add_tile_c2c<S, 16, 32, 4, 32, 32>(r, P);  // 64 us; 16x16x4 on 64 threads 74
   add_tile_c2c<S, 16, 64, 4, 32, 8, 8>(r, P);
-  // pass A (start: k_col 279 at 256, 325 at 1024)
+  // pass A (k_col: 279 at 256, 325 at 1024)
   add_tile_col<S, 32, 16, 32, 5, 16, 16>(r, P);  // 203; 64 registers spill: 239
   add_tile_col<S, 32, 16, 32, 4, 16, 32>(r, P);  // 212; 16x16x2: 227
   add_tile_col<S, 32, 16, 16, 4, 16, 32>(r, P);
   add_tile_col<S, 16, 32, 16, 4, 32, 32>(r, P);  // 227; 16x16x4 on 64 threads 238
   add_tile_col<S, 16, 64, 16, 4, 32, 8, 8>(r, P);  // 295; 8 columns a tile 335
-  // pass B (start: k_row 203 at 256, 262 at 1024)
+  // pass B (k_row: 203 at 256, 262 at 1024)
   add_tile_row<S, 32, 16, 8, 16, 16>(r, P);     // 179
   add_tile_row<S, 32, 32, 8, 16, 2, 16>(r, P);  // 187; 8x8x8 190
   add_tile_row<S, 16, 64, 8, 16, 4, 16>(r, P);  // 199; 32x32 212
