@@ -43,6 +43,16 @@ def input_size(plan: Plan) -> int:
     return _span(plan.in_count, L.istride, L.howmany, L.idist)
 
 
+def _target(numel, count, stride, howmany, dist, dtype, device):
+    """A buffer for a plan to write: zeros where the layout leaves gaps. A packed
+    or column layout without any is written in full, so it is not cleared first
+    (a fill of 8192 x 4096 f32 takes 20 us, the DCT-II that follows 121)."""
+    packed = stride == 1 and (howmany == 1 or dist == count)
+    columns = dist == 1 and stride == howmany
+    full = howmany > 0 and numel == count * howmany and (packed or columns)
+    return (torch.empty if full else torch.zeros)(numel, dtype=dtype, device=device)
+
+
 class PlanFunction(torch.autograd.Function):
     """y = plan(x) on flat device buffers laid out as the plan describes."""
 
@@ -51,7 +61,9 @@ class PlanFunction(torch.autograd.Function):
         if x.dtype != _side_dtype(plan, "in") or x.numel() < input_size(plan):
             raise ValueError("input buffer does not match the plan")
         x = x.contiguous()
-        y = torch.zeros(output_size(plan), dtype=_side_dtype(plan, "out"), device=x.device)
+        L = plan.layout
+        y = _target(output_size(plan), plan.out_count, L.ostride, L.howmany, L.odist,
+                    _side_dtype(plan, "out"), x.device)
         plan.execute_async(x, y, stream=torch.cuda.current_stream())
         ctx.plan = plan
         ctx.in_numel = x.numel()
@@ -61,7 +73,9 @@ class PlanFunction(torch.autograd.Function):
     def backward(ctx, gy: torch.Tensor):
         plan = ctx.plan
         gy = gy.contiguous()
-        gx = torch.zeros(ctx.in_numel, dtype=_side_dtype(plan, "in"), device=gy.device)
+        L = plan.layout
+        gx = _target(ctx.in_numel, plan.in_count, L.istride, L.howmany, L.idist,
+                     _side_dtype(plan, "in"), gy.device)
         plan.adjoint_async(gy, gx, stream=torch.cuda.current_stream())
         return gx, None
 
