@@ -17,8 +17,9 @@ struct RadixCost {
 };
 const RadixCost kRadix[] = {{16, 40}, {15, 43}, {13, 45}, {12, 38}, {11, 42}, {10, 39}, {9, 42},
                             {8, 36},  {7, 39},  {6, 36},  {5, 37},  {4, 33},  {3, 35},  {2, 32}};
-// per thread and stage: barriers, stage description, loop control
-constexpr double kStageOverhead = 150;
+// per thread and stage: barriers, stage description, loop control; and where
+// no other blocks hide the barriers and the LDS accesses
+constexpr double kStageOverhead = 150, kStageWait = 670;
 
 // the compiled shape of radix r with at least kb butterflies, or -1
 int shape_for(int r, int64_t kb, int pts) {
@@ -73,7 +74,7 @@ int conflicts(int slots, F &&addr) {
 }  // namespace
 
 bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int lanes,
-                 FlexDesc *out) {
+                 FlexDesc *out, const FlexWait *wait) {
   if (n < 2 || n >= (1 << 15)) return false;
   std::vector<std::vector<int>> sets;
   std::vector<int> cur;
@@ -86,9 +87,11 @@ bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int 
     for (int r : c)
       for (const auto &sh : kFlexShapes)
         if (sh.r == r) cand.insert((int)((n / r + sh.k - 1) / sh.k));
+    if (wait && wait->spare) cand.insert({2, 4, 8, 16});  // threads beyond the butterflies
     for (int tpt : cand) {
       if (tpt > block || tpt < 1) continue;
       double work = 0;
+      int first = 0;  // points of the first stage a thread
       bool ok = true;
       for (int r : c) {
         const int64_t nb = n / r;
@@ -97,22 +100,31 @@ bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int 
           ok = false;
           break;
         }
-        work += (double)kFlexShapes[sh].k * r * radix_cost(r) + kStageOverhead;
+        work += (double)kFlexShapes[sh].k * r * radix_cost(r) + (wait ? kStageWait : kStageOverhead);
+        if (r == c.front()) first = kFlexShapes[sh].k * r;
       }
       if (!ok) continue;
+      if (wait) work += wait->real * (2.0 * n / tpt) + wait->first * first;
       // members per block: the fullest waves among blocks of up to 512
       // threads (or one member), LDS permitting (half of a CU's, so that two
-      // blocks share it, where a block holds several members)
+      // blocks share it, where a block holds several members); a waiting
+      // batch takes one wave's members until the chip is full
       const int64_t mem = (n + n / 8 + 34) * csize;
       if ((n + 2) * csize > lds_max) continue;
       const int most = lanes ? lanes : 512;
       int tmax = std::min(most, std::max(1, std::min(block, lanes ? block : 512) / tpt));
       tmax = (int)std::min<int64_t>(tmax, std::max<int64_t>(1, std::min<int64_t>(lds_max, lds_max / 2) / mem));
-      for (int tpb = lanes ? tmax : 1; tpb <= tmax; ++tpb) {
+      const int least = lanes ? tmax : wait ? std::min(tmax, std::max(1, 64 / tpt)) : 1;
+      for (int tpb = least; tpb <= tmax; ++tpb) {
         const int threads = (tpt * tpb + 63) / 64 * 64;
         if (threads > block) break;
         double cost = work * threads / ((double)tpb * n);
-        if (!lanes && threads < 192) cost *= 1.0 + 0.1 * (192 - threads) / 64;  // few waves a block
+        if (wait) {
+          const int64_t all = (wait->members + tpb - 1) / tpb * threads;
+          cost = work * std::max(1.0, (double)all / wait->resident);
+        }
+        if (!lanes && !wait && threads < 192)
+          cost *= 1.0 + 0.1 * (192 - threads) / 64;  // few waves a block
         if (threads > 256) cost *= 1.03;                                       // wider barriers
         if (lanes) cost *= 1.0 + 0.5 * (lanes - tpb) / lanes;                  // shorter runs
         if (!best_tpt || cost < best) {

@@ -31,12 +31,12 @@ static const char *flex_kind_name(int k) {
 // The entry and chain for engine length m: the smallest block size that
 // holds a member. 20 points a thread in FP32 (92 registers), 16 in FP64.
 static const FlexEntry *flex_find(int kind, int64_t m, int prec, bool bwd, int lanes,
-                                  FlexDesc *d) {
+                                  FlexDesc *d, const FlexWait *wait = nullptr) {
   const int pts = prec_compute_bytes(prec) == 8 ? 16 : 20;
   const FlexEntry *big = nullptr;
   for (const auto &e : flex_registry()) {
     if (e.kind != kind || e.prec != prec || e.bwd != bwd) continue;
-    if (!lanes && flex_choose(m, pts, e.block, 2 * prec_compute_bytes(prec), 160 * 1024, 0, d))
+    if (!lanes && flex_choose(m, pts, e.block, 2 * prec_compute_bytes(prec), 160 * 1024, 0, d, wait))
       return &e;
     big = &e;
   }
@@ -47,6 +47,29 @@ static const FlexEntry *flex_find(int kind, int64_t m, int prec, bool bwd, int l
         return &e;
   }
   return nullptr;
+}
+
+// Real transforms move a member's reals or bins through LDS outside the chain.
+// The chain of least work per member leaves that to few threads (2 for a
+// DCT-II of 60), which a full chip hides and a small batch waits for: DCT-II
+// of 60 FP32, 256 members, 9.6 us, 6.6 on the runtime chain's 16 threads, and
+// 5.0 with 16 threads here; of 3000, 64 members, 13.8, 10.8 and 9.4. So a batch
+// of at most half the threads that the chip runs well at once takes the chain
+// of least predicted time (units of flex_chain.cpp's work, fitted to 4300
+// measured pairs of chains; the DCT-III also computes a bin in its first
+// loads). Above that line it is the slower one (DCT-II of 300 FP64, 2048
+// members: 13.7 against 10.2 us with 75 threads against 15), and members of
+// more than 2048 pairs have a hundred threads or more already (R2C of 12000:
+// 10.8 against 10.1 us). C2R moves its reals in the chain's own stages.
+static bool flex_wait(int kind, int64_t m, int prec, int64_t howmany, const FlexDesc &d,
+                      FlexWait *w) {
+  if (m > 2048 || (kind != FK_R2C && kind != FK_DCT2 && kind != FK_DCT3)) return false;
+  w->members = howmany;
+  w->resident = (int64_t)cu_count() * (prec_compute_bytes(prec) == 8 ? 256 : 512);
+  w->real = kind == FK_DCT2 ? 130 : 55;
+  w->first = kind == FK_DCT3 ? 300 : 0;
+  w->spare = kind != FK_R2C;  // its first loads come from memory: repeated, they cost time
+  return (howmany + d.tpb - 1) / d.tpb * flex_threads(d) <= w->resident / 2;
 }
 
 class FlexNode : public Node {
@@ -146,6 +169,11 @@ std::unique_ptr<Node> build_flex_node(const Problem &pp, std::string *why) {
   if (lanes && e && d.tpb < 4) e = nullptr;
   if (lanes && !e) e = flex_find(kind, m, p.prec, bwd, 0, &d);
   if (!e) return nullptr;
+  FlexWait w;
+  if (flex_wait(kind, m, p.prec, p.howmany, d, &w)) {
+    FlexDesc soon;
+    if (const FlexEntry *s = flex_find(kind, m, p.prec, bwd, 0, &soon, &w)) e = s, d = soon;
+  }
   const int64_t rb = prec_real_bytes(p.prec);
   const int64_t ie = kind == FK_C2C || kind == FK_C2R ? 2 * rb : rb;
   auto span = [&](int64_t dist, int64_t stride) {

@@ -81,6 +81,8 @@ struct PlanError {
 // no GPU implementation exists.
 std::unique_ptr<Node> build_node(const Problem &p, std::string *why);
 std::unique_ptr<Node> build_c2c_node(const Problem &p, std::string *why);
+// compute units of the current device (256 if it does not say)
+int cu_count();
 // C2C on the tile kernels (tile_plan.cpp); null, with *why untouched, where
 // they do not apply
 std::unique_ptr<Node> build_columns_node(const Problem &p, std::string *why);

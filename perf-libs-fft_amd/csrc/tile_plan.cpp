@@ -30,7 +30,7 @@ const std::vector<TileEntry> &tile_registry() {
   return reg;
 }
 
-static int cu_count() {
+int cu_count() {
   int dev = 0, c = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
