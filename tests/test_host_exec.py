@@ -232,11 +232,13 @@ def test_cosine_and_sine_transforms(exe, tmp_path, dtype):
 
 @pytest.mark.parametrize("dtype", ALL)
 def test_convolutions(exe, tmp_path, dtype):
-    # one block (Rader, Bluestein), three passes (Rader 12289, chirp-z 10007)
+    # one block (Rader, Bluestein), three passes (Rader 12289, chirp-z 10007 and
+    # 20011: rows of 96, 192 and 384 in FP64)
     run(exe, tmp_path, [P("c2c", n, hm, dtype, d, inplace=k)
                         for n, hm, d, k in ((17, 300, -1, 0), (97, 17, 1, 1), (59, 33, -1, 0),
                                             (509, 3, 1, 0), (1009, 2, -1, 1), (1399, 2, 1, 0),
-                                            (12289, 1, -1, 1), (10007, 2, 1, 0))])
+                                            (12289, 1, -1, 1), (10007, 2, 1, 0),
+                                            (20011, 1, -1, 0))])
 
 
 @pytest.mark.parametrize("dtype,direction,inplace", [("f32", -1, 0), ("f32", 1, 1), ("f64", -1, 0),
