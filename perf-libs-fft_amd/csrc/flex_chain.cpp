@@ -76,6 +76,7 @@ int conflicts(int slots, F &&addr) {
 bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int lanes,
                  FlexDesc *out, const FlexWait *wait) {
   if (n < 2 || n >= (1 << 15)) return false;
+  const bool idle = wait && wait->members > 0;
   std::vector<std::vector<int>> sets;
   std::vector<int> cur;
   multisets(n, 0, cur, sets);
@@ -100,11 +101,12 @@ bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int 
           ok = false;
           break;
         }
-        work += (double)kFlexShapes[sh].k * r * radix_cost(r) + (wait ? kStageWait : kStageOverhead);
+        work += (double)kFlexShapes[sh].k * r * radix_cost(r) + (idle ? kStageWait : kStageOverhead);
         if (r == c.front()) first = kFlexShapes[sh].k * r;
       }
       if (!ok) continue;
-      if (wait) work += wait->real * (2.0 * n / tpt) + wait->first * first;
+      if (wait)
+        work += wait->real * (2.0 * n / tpt) * (idle ? 1.0 : 1.0 + 8.0 / tpt) + wait->first * first;
       // members per block: the fullest waves among blocks of up to 512
       // threads (or one member), LDS permitting (half of a CU's, so that two
       // blocks share it, where a block holds several members); a waiting
@@ -114,16 +116,16 @@ bool flex_choose(int64_t n, int pts, int block, int csize, int64_t lds_max, int 
       const int most = lanes ? lanes : 512;
       int tmax = std::min(most, std::max(1, std::min(block, lanes ? block : 512) / tpt));
       tmax = (int)std::min<int64_t>(tmax, std::max<int64_t>(1, std::min<int64_t>(lds_max, lds_max / 2) / mem));
-      const int least = lanes ? tmax : wait ? std::min(tmax, std::max(1, 64 / tpt)) : 1;
+      const int least = lanes ? tmax : idle ? std::min(tmax, std::max(1, 64 / tpt)) : 1;
       for (int tpb = least; tpb <= tmax; ++tpb) {
         const int threads = (tpt * tpb + 63) / 64 * 64;
         if (threads > block) break;
         double cost = work * threads / ((double)tpb * n);
-        if (wait) {
+        if (idle) {
           const int64_t all = (wait->members + tpb - 1) / tpb * threads;
           cost = work * std::max(1.0, (double)all / wait->resident);
         }
-        if (!lanes && !wait && threads < 192)
+        if (!lanes && !idle && threads < 192)
           cost *= 1.0 + 0.1 * (192 - threads) / 64;  // few waves a block
         if (threads > 256) cost *= 1.03;                                       // wider barriers
         if (lanes) cost *= 1.0 + 0.5 * (lanes - tpb) / lanes;                  // shorter runs

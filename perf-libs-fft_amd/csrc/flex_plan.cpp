@@ -61,15 +61,27 @@ static const FlexEntry *flex_find(int kind, int64_t m, int prec, bool bwd, int l
 // members: 13.7 against 10.2 us with 75 threads against 15), and members of
 // more than 2048 pairs have a hundred threads or more already (R2C of 12000:
 // 10.8 against 10.1 us). C2R moves its reals in the chain's own stages.
+//
+// On a full chip the loads and stores of a DCT-II of 8 to 256 pairs count too,
+// per real and more the fewer lanes share a line (of 32, 2^19 members, FP32
+// 154 -> 57 us on 4 threads instead of one, FP64 314 -> 99; of 64, 2^18 members,
+// 144 -> 62). Shorter members lose (of 8, 2^21 members, 72 -> 81), longer ones
+// have ten threads and more, and in between, with more than half of the
+// resident threads but not all, least work per member is best (FP64 of 20,
+// 52428 members: 11.3 against 13.4).
 static bool flex_wait(int kind, int64_t m, int prec, int64_t howmany, const FlexDesc &d,
                       FlexWait *w) {
   if (m > 2048 || (kind != FK_R2C && kind != FK_DCT2 && kind != FK_DCT3)) return false;
-  w->members = howmany;
-  w->resident = (int64_t)cu_count() * (prec_compute_bytes(prec) == 8 ? 256 : 512);
-  w->real = kind == FK_DCT2 ? 130 : 55;
-  w->first = kind == FK_DCT3 ? 300 : 0;
-  w->spare = kind != FK_R2C;  // its first loads come from memory: repeated, they cost time
-  return (howmany + d.tpb - 1) / d.tpb * flex_threads(d) <= w->resident / 2;
+  const int64_t resident = (int64_t)cu_count() * (prec_compute_bytes(prec) == 8 ? 256 : 512);
+  const int64_t threads = (howmany + d.tpb - 1) / d.tpb * flex_threads(d);
+  if (threads > resident / 2) {
+    *w = FlexWait{0, 0, prec_compute_bytes(prec) == 8 ? 8.0 : 20.0, 0, false};
+    return kind == FK_DCT2 && m >= 8 && m <= 256 && threads >= resident;
+  }
+  // (R2C: its first loads come from memory; repeated by spare threads they cost time)
+  *w = FlexWait{howmany, resident, kind == FK_DCT2 ? 130.0 : 55.0, kind == FK_DCT3 ? 300.0 : 0.0,
+                kind != FK_R2C};
+  return true;
 }
 
 class FlexNode : public Node {
@@ -171,8 +183,8 @@ std::unique_ptr<Node> build_flex_node(const Problem &pp, std::string *why) {
   if (!e) return nullptr;
   FlexWait w;
   if (flex_wait(kind, m, p.prec, p.howmany, d, &w)) {
-    FlexDesc soon;
-    if (const FlexEntry *s = flex_find(kind, m, p.prec, bwd, 0, &soon, &w)) e = s, d = soon;
+    FlexDesc other;
+    if (const FlexEntry *o = flex_find(kind, m, p.prec, bwd, 0, &other, &w)) e = o, d = other;
   }
   const int64_t rb = prec_real_bytes(p.prec);
   const int64_t ie = kind == FK_C2C || kind == FK_C2R ? 2 * rb : rb;

@@ -1,6 +1,6 @@
 // Host check of the flexible chains chosen for least waiting time
-// (csrc/flex_chain.hpp, FlexWait): the replay of flex_chain_host.cpp over
-// small and large batches, and the threads a member gets: at least as many as
+// and with the work around them (csrc/flex_chain.hpp, FlexWait): the replay of
+// flex_chain_host.cpp over small, large and chip-filling batches, and the threads a member gets: at least as many as
 // for least work, and at most the butterflies or 16.
 #define main flex_chain_main
 #include "flex_chain_host.cpp"
@@ -13,6 +13,9 @@ int main() {
     for (int64_t n = 2; n <= 2048; ++n) {
       FlexDesc least, d;
       if (!flex_choose(n, c[0], c[1], c[2], 160 * 1024, 0, &least)) continue;
+      const FlexWait full = {0, 0, c[2] == 8 ? 20. : 8., 0, false};
+      CHECK(flex_choose(n, c[0], c[1], c[2], 160 * 1024, 0, &d, &full));
+      check(n, c[0], c[1], c[2], d);
       for (int64_t members : {1, 40, 1000, 30000})
         for (int kind = 0; kind < 3; ++kind) {
           const FlexWait w = {members, c[2] == 8 ? 131072 : 65536, kind == 1 ? 130. : 55.,
