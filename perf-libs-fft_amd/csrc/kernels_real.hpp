@@ -37,9 +37,12 @@ __device__ __forceinline__ cpx<typename ST::C> load_pair(const typename ST::Rs *
 // ---------------------------------------------------------------------------
 // Short packed members (at most 512 bytes): a thread's strided elements open a
 // line per few lanes. The block's members are consecutive: they are copied
-// through LDS with whole-line accesses on both sides. Bound by memory: R2C +
-// C2R of 2^24 reals as members of 64 in FP32 99 -> 68 us, FP64 68 -> 66 (half
-// as many); FP64 members of 128 (1 KB) are at 61 us without, 67 with.
+// through LDS with whole-line accesses on both sides. That pays once the batch
+// comes from HBM (flags bit 2, RealNode): 64 reals, R2C 2^17 members 20.1 ->
+// 18.3 us, 2^18 36.3 -> 34.6, C2R 18.7 -> 17.2 and 37.2 -> 33.8; below, the two
+// copies only add to a block's time (R2C 2^16 members 10.3 against 11.8, 4096
+// 4.2 against 5.2, C2R 8.9 against 11.4). The FP64 R2C's accesses are as wide
+// already (2^18 members: 53 us, 64 through LDS).
 // ---------------------------------------------------------------------------
 template <class Eng>
 constexpr bool short_real() {
@@ -80,9 +83,9 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
   const cpx<C> *W = static_cast<const cpx<C> *>(a.aux0);
   // flags bit1: interior bins doubled (the adjoint of C2R)
   const C h = (a.flags & 2) ? C(1) : C(0.5);
-  if constexpr (short_real<Eng>()) {
+  if constexpr (short_real<Eng>() && std::is_same_v<C, float>) {
     constexpr int M = Eng::NFIX, T = TPT * TPB;
-    if (pair_ok && os == 1 && a.idist == 2 * M && a.odist == M + 1) {
+    if ((a.flags & 4) && pair_ok && os == 1 && a.idist == 2 * M && a.odist == M + 1) {
       const int rows = (int)(a.count - tr + g < TPB ? a.count - tr + g : TPB);
       const int lper = Eng::lds_per(M);
       cpx<C> *all = dyn_lds<C>();
@@ -415,7 +418,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB)
   };
   if constexpr (short_real<Eng>() && Eng::REGS_IN) {
     constexpr int M = Eng::NFIX, T = TPT * TPB;
-    if (pair_ok && is == 1 && a.idist == M + 1 && a.odist == 2 * M) {
+    if ((a.flags & 4) && pair_ok && is == 1 && a.idist == M + 1 && a.odist == 2 * M) {
       using Ch = typename Eng::Ch;
       constexpr int R0 = Ch::radix(0), NB = M / R0, KB = (NB + TPT - 1) / TPT;
       const int rows = (int)(a.count - tr + g < TPB ? a.count - tr + g : TPB);

@@ -46,6 +46,10 @@ class RealNode : public Node {
   hipError_t init() {
     hipError_t err = eng_.init(c_, len());
     if (err != hipSuccess || !half_) return err;
+    // short packed members pass through LDS (kernels_real.hpp) once both sides
+    // together take 64 MiB (on 256 CUs), more than the caches keep
+    const int64_t bytes = batch_ * (2 * n_ + 2) * prec_real_bytes(prec_);
+    if (bytes >= (int64_t)cu_count() << 18) extra_ |= 4;
     return upload_table(aux_, root_table(n_, n_ / 2 + 1), prec_);
   }
   hipError_t enqueue(const void *in, void *out, void *, hipStream_t s) const override {

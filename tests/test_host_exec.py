@@ -215,8 +215,10 @@ def test_real_transforms(exe, tmp_path, dtype):
         for kind in ("r2c", "c2r"):
             cases += [P(kind, n, hm, dtype, lay=REAL_PAD[kind](n), inplace=1),
                       P(kind, n, hm, dtype, adjoint=1)]
-    for n, hm in ((16, 700), (64, 70), (128, 33), (4096, 3)):  # short members through LDS
+    for n, hm in ((16, 700), (64, 70), (128, 33), (4096, 3)):
         cases += [P("r2c", n, hm, dtype), P("c2r", n, hm, dtype)]
+    # (one CU: the line above which short members pass through LDS)
+    cases += [P(k, n, hm, dtype, cus=1) for n, hm in ((64, 1030), (128, 517)) for k in ("r2c", "c2r")]
     cases += [P("r2c", 100, 5, dtype, lay=(2, 211, 1, 53)), P("c2r", 100, 5, dtype, lay=(1, 53, 3, 301))]
     run(exe, tmp_path, cases)
 
