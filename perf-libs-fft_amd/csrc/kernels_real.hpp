@@ -146,7 +146,10 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
       const int k = t + i * TPT;
       wk[i] = (2 * k <= NF) ? W[k] : cpx<C>{C(0), C(0)};
     }
-    auto body = [&](auto pair, auto unit) {
+    // guard: absent members load nothing. For a block with members missing and
+    // strided reals, whose loads are a line each: one member of 512 to 4096
+    // reals at stride 2 5.9 -> 4.6 us and 6.7 -> 5.9; full blocks lose 12 %.
+    auto body = [&](auto pair, auto unit, auto guard) {
       constexpr bool U = decltype(unit)::value;
       Eng::template run<true>(
           a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
@@ -154,6 +157,7 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
             if constexpr (decltype(pair)::value) {
               return ST::ld(reinterpret_cast<const E *>(x)[b + o]);
             } else {
+              if (decltype(guard)::value && !valid) return cpx<C>{C(0), C(0)};
               const Rs *p = x + (int64_t)(2 * b) * is + (int64_t)(2 * o) * is;
               return cpx<C>{ST::ldr(p[0]), ST::ldr(p[is])};
             }
@@ -166,9 +170,10 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_r2c_even(KArgs a) {
         if (2 * k <= NF) post(k, wk[i], U ? int64_t(1) : os);
       }
     };
-    if (pair_ok && os == 1) body(std::true_type{}, std::true_type{});
-    else if (pair_ok) body(std::true_type{}, std::false_type{});
-    else body(std::false_type{}, std::false_type{});
+    if (pair_ok && os == 1) body(std::true_type{}, std::true_type{}, std::false_type{});
+    else if (pair_ok) body(std::true_type{}, std::false_type{}, std::false_type{});
+    else if (a.count < TPB) body(std::false_type{}, std::false_type{}, std::true_type{});
+    else body(std::false_type{}, std::false_type{}, std::false_type{});
   } else {
     Eng::template run<true>(
         a.desc, lds, static_cast<const cpx<C> *>(a.tw), t, valid,
@@ -479,10 +484,17 @@ __global__ void __launch_bounds__(Eng::TPT *TPB)
     constexpr int NB = NF / R0;
     constexpr int KB = (NB + TPT - 1) / TPT;
     cpx<C> vin[KB * R0];
+    // Members of 16 points a thread on one wave or less: one predicate over a
+    // thread's bins, without which the scheduler raises 62 registers to 76 and
+    // absent members load as well. C2R of 512: one member 5.2 -> 4.4 us, 4096
+    // 7.3 -> 6.0, at stride 2 11.3 -> 7.5; the longer and the FP64 kernels are
+    // up to 5 % slower with it.
+    constexpr bool kGuard = std::is_same_v<C, float> && R0 == 16 && TPT <= 16;
     auto build = [&](auto unit) {
       constexpr bool U = decltype(unit)::value;  // unit input stride
 #pragma unroll
       for (int k = 0; k < KB; ++k) {
+        if (kGuard && !valid) break;
         int b = t + k * TPT;
         if (NB % TPT != 0) b = b < NB ? b : NB - 1;
         const cpx<C> wb = W[b];
@@ -792,6 +804,9 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_dct3_even(KArgs a) {
     cpx<C> vin[KB * R0];
 #pragma unroll
     for (int k = 0; k < KB; ++k) {
+      // (the predicate keeps 87 registers where 123 would hold all of a
+      // thread's bins: 4096 members of 4096 reals at stride 2 63.4 -> 53.4 us)
+      if (!valid) break;
       int b = t + k * TPT;
       if (NB % TPT != 0) b = b < NB ? b : NB - 1;
       const cpx<C> Wb = W[b], wb = w[b];

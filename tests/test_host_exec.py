@@ -219,6 +219,8 @@ def test_real_transforms(exe, tmp_path, dtype):
         cases += [P("r2c", n, hm, dtype), P("c2r", n, hm, dtype)]
     # (one CU: the line above which short members pass through LDS)
     cases += [P(k, n, hm, dtype, cus=1) for n, hm in ((64, 1030), (128, 517)) for k in ("r2c", "c2r")]
+    cases += [P("r2c", 512, hm, dtype, lay=(2, 1025, 1, 257)) for hm in (1, 17)]
+    cases += [P("c2r", 512, hm, dtype, lay=(2, 515, 1, 512)) for hm in (1, 17)]
     cases += [P("r2c", 100, 5, dtype, lay=(2, 211, 1, 53)), P("c2r", 100, 5, dtype, lay=(1, 53, 3, 301))]
     run(exe, tmp_path, cases)
 
