@@ -103,31 +103,31 @@ static hipError_t bluestein_kernel(int64_t n, int64_t M, const std::vector<doubl
 }
 
 // [j][i], j < rows, i < count: W_M^{j step i}; transposed: [i][j]
-static void cz_table(std::vector<double> *t, int64_t M, int64_t rows, int64_t count,
-                     int64_t step, bool transposed) {
+static void cz_table(std::vector<double> *t, const SplitRoots &root, int64_t M, int64_t rows,
+                     int64_t count, int64_t step, bool transposed) {
   const int64_t no = transposed ? count : rows, ni = transposed ? rows : count;
+  const size_t at = t->size();
+  t->resize(at + 2 * (size_t)(no * ni));
+  double *out = t->data() + at;
   for (int64_t o = 0; o < no; ++o)
-    for (int64_t i = 0; i < ni; ++i) {
-      double re, im;
-      unit_root(o * i * step % M, M, &re, &im);
-      t->push_back(re);
-      t->push_back(-im);
-    }
+    for (int64_t i = 0; i < ni; ++i, out += 2) root(o * i * step % M, out);
 }
 
 std::vector<double> cz_mid_twiddles(int64_t n1, const Choice &mid) {
   const int64_t n2 = mid.e->n, R = mid.chain[0], NB = n2 / R, M = n1 * n2;
+  const SplitRoots root(M);
   std::vector<double> t;
-  cz_table(&t, M, n1, NB, 1, false);
-  cz_table(&t, M, n1, R, NB, false);
+  cz_table(&t, root, M, n1, NB, 1, false);
+  cz_table(&t, root, M, n1, R, NB, false);
   return t;
 }
 
 std::vector<double> cz_col_twiddles(const Choice &col, int64_t n2) {
   const int64_t n1 = col.e->n, R = col.chain.back(), NB = n1 / R, M = n1 * n2;
+  const SplitRoots root(M);
   std::vector<double> t;
-  cz_table(&t, M, n2, NB, 1, true);
-  cz_table(&t, M, n2, R, NB, true);
+  cz_table(&t, root, M, n2, NB, 1, true);
+  cz_table(&t, root, M, n2, R, NB, true);
   return t;
 }
 

@@ -190,6 +190,23 @@ hipError_t dft_f64_gpu(std::vector<double> &v, int64_t M, int64_t count);
 void unit_root(int64_t num, int64_t den, double *re, double *im);
 void unit_root_l(int64_t num, int64_t den, long double *re, long double *im);
 
+// Many roots of one order n: W_n^e = exp(-2 pi i e/n), 0 <= e < n, as the
+// product of two roots held in long double (2 sqrt(n) of them), rounded once:
+// 4 ns against 70 for a cosine and a sine, the same half unit in the last place.
+class SplitRoots {
+ public:
+  explicit SplitRoots(int64_t n);
+  void operator()(int64_t e, double *out) const {
+    const long double *l = &lo_[2 * (e & (((int64_t)1 << shift_) - 1))], *h = &hi_[2 * (e >> shift_)];
+    out[0] = (double)(l[0] * h[0] - l[1] * h[1]);
+    out[1] = (double)-(l[0] * h[1] + l[1] * h[0]);
+  }
+
+ private:
+  int shift_;
+  std::vector<long double> lo_, hi_;
+};
+
 // Last error text for the calling thread (plan creation diagnostics).
 void set_last_error(const std::string &s);
 const char *last_error();

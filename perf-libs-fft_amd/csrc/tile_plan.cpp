@@ -117,20 +117,9 @@ class TileFourStepNode : public Node {
     if (err == hipSuccess) err = upload_table(tw2_, stockham_twiddles(row_->chain), p_.prec);
     if (err != hipSuccess) return err;
     // T1[c][b] = W_N^{c b} (b < NB) and T2[c][m] = W_N^{c NB m} (m < RL), each
-    // rounded once: products of split roots taken in long double
+    // rounded once
     const int64_t n = n1_ * n2_, RL = col_->chain.back(), NB = n1_ / RL;
-    int lg = 0;
-    while ((int64_t(1) << lg) < n) ++lg;
-    const int shift = (lg + 1) / 2;
-    const int64_t nlo = int64_t(1) << shift, nhi = ((n - 1) >> shift) + 1;
-    std::vector<long double> lo(2 * nlo), hi(2 * nhi);
-    for (int64_t r = 0; r < nlo; ++r) unit_root_l(r, n, &lo[2 * r], &lo[2 * r + 1]);
-    for (int64_t q = 0; q < nhi; ++q) unit_root_l(q * nlo, n, &hi[2 * q], &hi[2 * q + 1]);
-    auto root = [&](int64_t e, double *out) {  // forward sign
-      const long double *l = &lo[2 * (e & (nlo - 1))], *h = &hi[2 * (e >> shift)];
-      out[0] = (double)(l[0] * h[0] - l[1] * h[1]);
-      out[1] = (double)-(l[0] * h[1] + l[1] * h[0]);
-    };
+    const SplitRoots root(n);
     std::vector<double> t1(2 * n2_ * NB), t2(2 * n2_ * RL);
     for (int64_t c = 0; c < n2_; ++c) {
       for (int64_t b = 0; b < NB; ++b) root(c * b, &t1[2 * (c * NB + b)]);

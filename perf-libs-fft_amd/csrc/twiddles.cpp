@@ -49,6 +49,17 @@ void unit_root(int64_t num, int64_t den, double *re, double *im) {
   *im = (double)s;
 }
 
+SplitRoots::SplitRoots(int64_t n) {
+  int lg = 0;
+  while ((int64_t(1) << lg) < n) ++lg;
+  shift_ = (lg + 1) / 2;
+  const int64_t nlo = int64_t(1) << shift_, nhi = ((n - 1) >> shift_) + 1;
+  lo_.resize(2 * nlo);
+  hi_.resize(2 * nhi);
+  for (int64_t r = 0; r < nlo; ++r) unit_root_l(r, n, &lo_[2 * r], &lo_[2 * r + 1]);
+  for (int64_t q = 0; q < nhi; ++q) unit_root_l(q * nlo, n, &hi_[2 * q], &hi_[2 * q + 1]);
+}
+
 std::vector<double> stockham_twiddles(const std::vector<int> &chain) {
   std::vector<double> tw;
   int64_t L = chain.empty() ? 1 : chain[0];
