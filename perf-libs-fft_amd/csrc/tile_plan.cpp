@@ -87,14 +87,21 @@ class TileColumnsNode : public Node {
 
 // Members closer together than their elements on both sides: lanes along the
 // members (a line holds up to 16 of them) instead of along the elements (a
-// line each). Below a quarter of the chip's CUs in tiles the general kernel's
-// smaller blocks are faster: 1024 points FP32, 6.9 against 8.7 us for 100
-// columns (7 tiles), 15.0 against 9.6 for 1024 (64 tiles), 219 against 65 for
-// 16384.
+// line each). Few tiles wait for the block's chain, and the general kernel's
+// smaller blocks may be faster: below a quarter of the chip's CUs in tiles for 64
+// and 512 points, an eighth in FP64 and for 2048, else a 32nd. In us, general
+// kernel and tiles, on 8 / 16 / 32 tiles: FP32 128 points 6.1 4.4 / 6.2 4.4 / 6.3
+// 4.4, 256 6.2 5.3 / 6.3 5.4 / 6.4 5.5, 512 7.0 8.1 / 7.1 8.3 / 7.5 8.3, 1024
+// 10.6 8.6 / 11.1 8.9 / 11.5 9.2, 2048 13.6 18.1 / 15.5 18.5 / 22.6 19.1; FP64
+// 256 5.0 4.6 / 5.1 4.7 / 5.1 4.8, 512 5.6 7.6 / 5.7 7.8 / 6.6 7.9, 1024 7.8 7.9 /
+// 8.1 8.4 / 9.3 9.0; f16 64 4.2 4.9 / 4.2 5.0 / 4.2 5.0, 512 7.4 9.7 / 8.0 9.8 /
+// 9.7 9.7, 1024 13.1 10.3 / 14.6 11.6 / 18.6 13.7; 64 points FP32 and FP64 alike.
 std::unique_ptr<Node> build_columns_node(const Problem &p, std::string *why) {
   if (p.howmany < 2 || p.idist >= p.istride || p.odist >= p.ostride) return nullptr;
   const TileEntry *e = find_tile(TK_C2C, p.n, p.prec, p.dir > 0);
-  if (!e || (p.howmany + e->w - 1) / e->w < cu_count() / 4) return nullptr;
+  if (!e) return nullptr;
+  const int share = p.n == 64 || p.n == 512 ? 4 : p.n == 2048 || p.prec == P_F64 ? 8 : 32;
+  if ((p.howmany + e->w - 1) / e->w < cu_count() / share) return nullptr;
   auto node = std::make_unique<TileColumnsNode>(e, p);
   const hipError_t err = node->init();
   if (err != hipSuccess) {
@@ -204,8 +211,10 @@ class TileFourStepNode : public Node {
 // thread of kernels.hpp answer sooner (2^18 FP32: 19 against 26 us for 4
 // members, 24 against 27 for 8 (128 blocks), 68 against 52 for 32; 2^18 FP64:
 // 21 against 23 us for 4, 34 against 33 for 8 (256 blocks)). The 16-bit types
-// have only runtime chains there (65536: 22 against 12 us for one member,
-// 738 against 167 for 512).
+// have only runtime chains there and always take the tiles (f16, passes against
+// tiles: 65536 17.3 and 12.4 us for one member, 22.1 and 14.5 for 16, 59.6 and
+// 25.9 for 64; 2^18 24.6 and 22.0, 32 and 26 for 8, 216 and 91 for 64; 2^20 36.8
+// and 23.7, 642 and 401 for 64).
 std::unique_ptr<Node> build_tile_fourstep_node(const Problem &p, std::string *why) {
   for (const auto &row : tile_registry()) {
     if (row.kind != TK_ROW || row.prec != p.prec || row.bwd != (p.dir > 0)) continue;
