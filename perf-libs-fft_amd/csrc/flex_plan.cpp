@@ -172,13 +172,20 @@ std::unique_ptr<Node> build_flex_node(const Problem &pp, std::string *why) {
     else if (p.r2r_kind == 2 || p.r2r_kind == 6) kind = FK_DCT3, bwd = p.r2r_kind == 6;
     else return nullptr;
   }
-  // columns: lanes along the members that share a line
+  // columns: lanes along the members that share a line. Fewer than eight members
+  // fill half a line at most (us without and with, FP32: 360 points 5.6 and 6.5
+  // for 4 members, 6.0 and 6.5 for 8; 100 points 5.6 and 4.4 for 8; 1500 11.4 and
+  // 8.1). Long members that leave a block two or three of them wait for it until
+  // there are some 64 (3000 points FP32 17.0 and 17.6 for 32, 19.1 and 17.3 for
+  // 64, 43.6 and 27.9 for 512, 307 and 191 for 4096; 2000 points FP64 7.8 and 9.4
+  // for 8, 12.5 and 9.9 for 64, 70 and 48 for 1024); with one there is nothing to
+  // share.
   const int lanes = kind == FK_C2C && p.howmany >= 8 && p.idist < p.istride && p.odist < p.ostride
                         ? 128 / (2 * prec_compute_bytes(p.prec))
                         : 0;
   FlexDesc d;
   const FlexEntry *e = flex_find(kind, m, p.prec, bwd, lanes, &d);
-  if (lanes && e && d.tpb < 4) e = nullptr;
+  if (lanes && e && (d.tpb < 2 || (d.tpb < 4 && p.howmany < 64))) e = nullptr;
   if (lanes && !e) e = flex_find(kind, m, p.prec, bwd, 0, &d);
   if (!e) return nullptr;
   FlexWait w;

@@ -204,6 +204,8 @@ def test_flexible_chains(exe, tmp_path, dtype):
     cases += [P("c2c", 100, 149, dtype, -1, "cols", node="lanes"),
               P("c2c", 60, 33, dtype, 1, (35, 1, 33, 1), node="lanes"),
               P("c2c", 1000, 17, dtype, 1, "cols", inplace=1, node="lanes"),
+              # two and three members a block
+              P("c2c", {"f64": 2000}.get(dtype, 3000), 65, dtype, -1, "cols", node="lanes"),
               P("c2c", 360, 9, dtype, -1, (2, 725, 3, 1081))]
     run(exe, tmp_path, cases)
 
