@@ -289,10 +289,10 @@ class BigBluesteinNode : public Node {
 // Each member's workspace is M complex values of the compute precision.
 class ChirpZ3Node : public Node {
  public:
-  ChirpZ3Node(int64_t n, int64_t n1, int64_t n2, int prec, bool bwd, int64_t batch, int64_t is,
+  ChirpZ3Node(int64_t n, int64_t n1, int64_t n2, int prec, int64_t batch, int64_t is,
               int64_t id, int64_t os, int64_t od, int64_t chunk, Choice cin, Choice cmid,
               Choice cout)
-      : n_(n), n1_(n1), n2_(n2), prec_(prec), bwd_(bwd), batch_(batch), is_(is), id_(id),
+      : n_(n), n1_(n1), n2_(n2), prec_(prec), batch_(batch), is_(is), id_(id),
         os_(os), od_(od), chunk_(chunk), cin_(std::move(cin)), cmid_(std::move(cmid)),
         cout_(std::move(cout)) {}
   hipError_t init() {
@@ -389,7 +389,6 @@ class ChirpZ3Node : public Node {
  private:
   int64_t n_, n1_, n2_;
   int prec_;
-  bool bwd_;
   int64_t batch_, is_, id_, os_, od_, chunk_;
   Choice cin_, cmid_, cout_;
   EngineData ein_, emid_, eout_;
@@ -403,10 +402,10 @@ class ChirpZ3Node : public Node {
 // workspace is N complex values, then two slots per member of the chunk.
 class Rader3Node : public Node {
  public:
-  Rader3Node(int64_t n, int64_t n1, int64_t n2, int prec, bool bwd, int64_t batch, int64_t is,
+  Rader3Node(int64_t n, int64_t n1, int64_t n2, int prec, int64_t batch, int64_t is,
              int64_t id, int64_t os, int64_t od, int64_t chunk, Choice cin, Choice cmid,
              Choice cout)
-      : n_(n), n1_(n1), n2_(n2), prec_(prec), bwd_(bwd), batch_(batch), is_(is), id_(id),
+      : n_(n), n1_(n1), n2_(n2), prec_(prec), batch_(batch), is_(is), id_(id),
         os_(os), od_(od), chunk_(chunk), cin_(std::move(cin)), cmid_(std::move(cmid)),
         cout_(std::move(cout)) {}
   hipError_t init() {
@@ -491,9 +490,11 @@ class Rader3Node : public Node {
         err = cmid_.e->launch(a, a.count / cmid_.e->tpb, cmid_.e->lds_bytes(n2_), s);
       }
       // 3. permuted-output columns, one block per CU: the scattered stores
-      // of fewer members in flight stay in L2 until their lines fill
-      // (65537, batch 2047: 1.44 -> 1.03 ms in f32; 2.28 -> 2.08 ms for the
-      // f64 plan). The launch asks for more than half of the CU's 160 KB LDS.
+      // of fewer members in flight stay in L2 until their lines fill. The launch
+      // asks for more than half of the CU's 160 KB LDS. 65537 in us by what it
+      // asks for (its own need, 41 KB, 54 KB, this): f32 512 members 664, 645,
+      // 592, 590, 2048 members 2787, 2548, 2389, 2339; f64 256 members 520, 523,
+      // 507, 466; f16 512 members 535, 538, 518, 545.
       if (err == hipSuccess) {
         a.in = work;
         a.out = static_cast<char *>(out) + (size_t)(b0 * od_) * eb;
@@ -522,7 +523,6 @@ class Rader3Node : public Node {
  private:
   int64_t n_, n1_, n2_;
   int prec_;
-  bool bwd_;
   int64_t batch_, is_, id_, os_, od_, chunk_;
   Choice cin_, cmid_, cout_;
   EngineData ein_, emid_, eout_;
@@ -645,7 +645,7 @@ std::unique_ptr<Node> build_bluestein(const Problem &p, std::string *why) {
     if (rd3_choice(p.n - 1, p.prec, bwd, &n1, &ci, &cm, &co)) {
       const int64_t N = p.n - 1;
       const int64_t chunk = fourstep_chunk(N, p.prec, p.howmany);
-      auto node = std::make_unique<Rader3Node>(p.n, n1, N / n1, p.prec, bwd, p.howmany,
+      auto node = std::make_unique<Rader3Node>(p.n, n1, N / n1, p.prec, p.howmany,
                                                p.istride, id, p.ostride, od, chunk, ci, cm, co);
       const hipError_t err = node->init();
       if (err != hipSuccess) {
@@ -661,7 +661,7 @@ std::unique_ptr<Node> build_bluestein(const Problem &p, std::string *why) {
     Cz3Choice cz;
     if (cz3_choice(p.n, p.prec, bwd, &cz)) {
       const int64_t chunk = fourstep_chunk(cz.M, p.prec, p.howmany);
-      auto node = std::make_unique<ChirpZ3Node>(p.n, cz.n1, cz.M / cz.n1, p.prec, bwd,
+      auto node = std::make_unique<ChirpZ3Node>(p.n, cz.n1, cz.M / cz.n1, p.prec,
                                                 p.howmany, p.istride, id, p.ostride, od, chunk,
                                                 cz.cin, cz.cmid, cz.cout);
       const hipError_t err = node->init();

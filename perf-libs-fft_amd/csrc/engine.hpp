@@ -107,12 +107,10 @@ struct StaticEngine {
   static constexpr int LDS_PER = lds_padded<PAD>(N);
   static constexpr bool USES_LDS = NS > 1;
 
-  template <int SI, bool TO_LDS, bool LDS_IN, class Load, class Store, bool REGS_IN = false,
-            bool KEEP = false>
+  template <int SI, bool TO_LDS, bool LDS_IN, class Load, class Store, bool REGS_IN = false>
   static __device__ __forceinline__ void stage(cpx<C> *lds, const cpx<C> *__restrict__ tw,
                                                int t, bool valid, Load &load, Store &store,
-                                               const cpx<C> *vin = nullptr,
-                                               cpx<C> *keep = nullptr) {
+                                               const cpx<C> *vin = nullptr) {
     constexpr int R = Ch::radix(SI);
     constexpr int L = Ch::L(SI);
     constexpr int NB = N / R;
@@ -155,10 +153,7 @@ struct StaticEngine {
     for (int k = 0; k < KB; ++k) {
       const int b = bidx(k);
       const bool act = (NB % TPT == 0) || (b < NB);
-      if constexpr (LAST && KEEP) {
-#pragma unroll
-        for (int m = 0; m < R; ++m) keep[k * R + m] = v[k][m];
-      } else if constexpr (LAST && !TO_LDS) {
+      if constexpr (LAST && !TO_LDS) {
         if (act && valid) {
 #pragma unroll
           for (int m = 0; m < R; ++m) call_store(store, b, m * NB, v[k][m]);
@@ -178,9 +173,7 @@ struct StaticEngine {
       }
     }
     if constexpr (!LAST || TO_LDS) __syncthreads();
-    if constexpr (!LAST)
-      stage<SI + 1, TO_LDS, false, Load, Store, false, KEEP>(lds, tw, t, valid, load, store,
-                                                             nullptr, keep);
+    if constexpr (!LAST) stage<SI + 1, TO_LDS, false>(lds, tw, t, valid, load, store);
   }
 
   // Results stay in LDS (natural order, lds[lds_pad(e)]) when TO_LDS. With
@@ -192,7 +185,8 @@ struct StaticEngine {
   }
 
   // Stage 0 takes its inputs from registers: vin[k * R0 + m] holds element
-  // b + m * (N / R0) of butterfly b = t + k * TPT (zero where b >= N / R0).
+  // b + m * (N / R0) of butterfly b = t + k * TPT; what it holds for b >= N / R0
+  // is computed with and dropped.
   // Lets a caller issue the next member's loads before this member's stages,
   // or compute stage-0 inputs with knowledge of the butterfly they feed.
   // With TO_LDS the results stay in LDS as for run<true>.
@@ -202,17 +196,6 @@ struct StaticEngine {
                                                   bool valid = true) {
     auto none = [](int) { return cpx<C>{C(0), C(0)}; };
     stage<0, TO_LDS, false, decltype(none), Store, true>(lds, tw, t, valid, none, store, vin);
-  }
-
-  // run_regs with the last stage's outputs left in registers:
-  // keep[k * RL + m] = element b + m * (N / RL) of butterfly b = t + k * TPT
-  // (RL the last radix). Other threads may still read LDS on return.
-  static __device__ __forceinline__ void run_regs_keep(const cpx<C> *vin, cpx<C> *lds,
-                                                       const cpx<C> *tw, int t, cpx<C> *keep) {
-    auto none = [](int) { return cpx<C>{C(0), C(0)}; };
-    auto drop = [](int, cpx<C>) {};
-    stage<0, false, false, decltype(none), decltype(drop), true, true>(lds, tw, t, true, none,
-                                                                       drop, vin, keep);
   }
 };
 

@@ -1,6 +1,5 @@
 // kernels_f32_cz.hip -- three-pass chirp-z and Rader kernels with FP32 arithmetic
-// (f32, f16 and bf16 storage; the column and row engines of the four-step
-// passes, sides 64..1024).
+// (kernels_cz.hpp; f32, f16 and bf16 storage), sides 64..1024.
 #include "kernels_cz.hpp"
 #include "launch.hpp"
 

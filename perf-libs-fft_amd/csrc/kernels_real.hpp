@@ -386,7 +386,8 @@ __global__ void __launch_bounds__(Eng::TPT *TPB) k_c2r_even_split(KArgs a) {
 // ---------------------------------------------------------------------------
 // Compile-time chains: a register cap keeps the scheduler from holding all of a
 // thread's 2 R0 bins before the first is used (98 registers for 16 x 16 in
-// FP32, where 57 do); loads in bursts of four cost the long chains 3 to 6 %.
+// FP32, where 62 do); the split 4096-point kernel has 76 with and without it.
+// Loads in bursts of four cost the long chains 3 to 6 %.
 template <typename S, class Eng>
 constexpr int c2r_waves() {
   if (Eng::NFIX == 0) return 1;
