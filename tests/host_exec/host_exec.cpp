@@ -13,6 +13,7 @@
 // Input (stdin), a case a line: fields, then the files that hold the input and
 // receive the output of each order:
 //   plan  name kind n howmany dtype dir r2r is id os od adjoint inplace bytes in out
+//         (no bytes: the plan is described only)
 //   mixed name count dtype dir inplace lengths bytes in out
 //   fault which path   (a small kernel with a fault that must be found)
 // Sizes and the values are the caller's (test_host_exec.py).
@@ -291,7 +292,7 @@ void run_plan(std::istringstream &l) {
   plfft_plan_describe(p, buf, sizeof(buf));
   std::printf("%s %s\n", name.c_str(), buf);
   std::fflush(stdout);
-  in_three_orders(name, in, out, (size_t)bytes, inplace, [&](void *di, void *dout) {
+  if (bytes) in_three_orders(name, in, out, (size_t)bytes, inplace, [&](void *di, void *dout) {
     const plfft_status_t e = adjoint
                                  ? plfft_plan_execute_adjoint_async(p, di, dout, nullptr, nullptr)
                                  : plfft_plan_execute_async(p, di, dout, nullptr, nullptr);

@@ -253,3 +253,36 @@ def test_mixed_batches(exe, tmp_path, dtype, direction, inplace):
     lengths = prng.mixed_lengths(7, 24, hi=20000) + [1, 2, 4096, 8192, 10007, 3 * 1009, 2 * 1999]
     run(exe, tmp_path, [dict(lengths=lengths, dtype=dtype, direction=direction, inplace=inplace,
                              cus=c) for c in (256, 2)])
+
+
+def describe(exe, kind, n, howmany, dtype, lay):
+    line = f"plan c {kind} {n} {howmany} {dtype} -1 0 {' '.join(map(str, lay))} 0 0 0 - -\n"
+    r = subprocess.run([exe], input=line, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return r.stdout.split(" ", 1)[1]
+
+
+# kind, length, output distance, what bounds the input side (elements of one or two reals), types
+LIMITED = [(k, n, od, w, dt) for k, n, od, w, types in
+           (("c2c", 1000, 1000, 2, ("f32", "f64", "f16")), ("r2c", 1000, 501, 1, ("f32", "f64")),
+            ("c2r", 1000, 1000, 2, ("f32", "f64")), ("c2c", 256, 256, 2, ("f32", "f16")),
+            ("c2c", 1024, 1024, 2, ("f32", "f16")))
+           for dt in types]
+
+
+@pytest.mark.parametrize("kind,n,od,w,dtype", LIMITED)
+def test_distances_beyond_32_bit_offsets(exe, kind, n, od, w, dtype):
+    """A block's members are addressed with 32-bit byte offsets: from the first
+    distance on whose block reaches 2^32 bytes another kernel is chosen."""
+    def name(idist, odist):
+        return describe(exe, kind, n, 100000, dtype, (1, idist, 1, odist)).split()[0]
+
+    near = name(2 * n, od)
+    assert "flex" in near or "unit" in near
+    tpb = int(near.split("_b")[1].split("_")[0])
+    assert tpb > 1
+    # the distance at which the block's end lies at 2^32 bytes
+    last = 2 ** 32 // (w * np.dtype(STORE[dtype]).itemsize * tpb)
+    assert name(last - 2 * n, od) == near and name(last, od) != near
+    if kind == "c2c":
+        assert name(2 * n, last - 2 * n) == near and name(2 * n, last) != near
