@@ -624,6 +624,14 @@ std::unique_ptr<Node> build_bluestein(const Problem &p, std::string *why) {
   int64_t P2 = 1;
   while (P2 < 2 * p.n - 2) P2 *= 2;
   Choice c = choose(KK_BLUE, P2, p.prec, bwd);
+  // A batch that gives at most half of the CUs a block waits for one member's
+  // stages: more threads a member where there are such kernels. FP64 in us, 8
+  // points a thread and 16: M = 128 4.6 and 6.0 for one member, 5.9 and 7.4 for
+  // 4096 (128 blocks), 22.9 and 23.4 for 32768; M = 1024 6.8 and 7.4, 7.8 and 8.8
+  // for 512 (128 blocks), 10.6 and 9.8 for 1024; M = 2048 7.0 and 8.6, 8.0 and 9.8
+  // for 256 (128 blocks), 15.5 and 15.0 for 1024, 105 and 89 for 8192.
+  if (c.e && c.e->n && (p.howmany + c.e->tpb - 1) / c.e->tpb * 2 <= cu_count())
+    c = choose(KK_BLUE, P2, p.prec, bwd, 0, false, true);
   int64_t M = P2;
   if (!c.e || !c.e->n) {
     int64_t S = 2 * p.n - 2;

@@ -14,6 +14,10 @@ void register_kernels_conv_f64(std::vector<KEntry> &r) {
     PLF_BLUE_TILE(S, P,   64,   4, 16, 4, 16);
     PLF_BLUE_TILE(S, P,  128,   2, 16, 8, 16);
     PLF_BLUE_TILE(S, P,  256,   1, 16, 16, 16);
+    // 8 points a thread, for few members (build_bluestein)
+    PLF_BLUE_TILE(S, P,   16,  16, 8, 2, 8);
+    PLF_BLUE_TILE(S, P,  128,   2, 8, 2, 8, 8);
+    PLF_BLUE_TILE(S, P,  256,   1, 8, 4, 8, 8);
     PLF_DYNAMIC(k_bluestein, KK_BLUE, S, P,  64,   4, 16);
     PLF_DYNAMIC(k_bluestein, KK_BLUE, S, P, 256,   1, 16);
     PLF_DYNAMIC(k_bluestein, KK_BLUE, S, P, 1024,  1, 8);

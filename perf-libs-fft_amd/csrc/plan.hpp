@@ -112,7 +112,7 @@ struct Choice {
 // packed: members contiguous at distance n with unit stride (cross-lane
 // kernels need it)
 Choice choose(int kind, int64_t len, int prec, bool bwd, int need_tpb_div = 0,
-              bool packed = false);
+              bool packed = false, bool few = false);
 std::vector<int> dynamic_chain(int64_t n);
 std::string chain_str(const Choice &c);
 // Upload a FP64 table (interleaved re/im) in the compute precision.

@@ -120,9 +120,11 @@ std::vector<int> dynamic_chain(int64_t n) {
   return c;
 }
 
-// Compile-time chain first (registry order = preference), else the dynamic
-// entry with the fewest threads that fits.
-Choice choose(int kind, int64_t len, int prec, bool bwd, int need_tpb_div, bool packed) {
+// Compile-time chain first (registry order = preference; for few members the
+// one with the most threads a member), else the dynamic entry with the fewest
+// threads that fits.
+Choice choose(int kind, int64_t len, int prec, bool bwd, int need_tpb_div, bool packed,
+              bool few) {
   Choice c;
   std::vector<Choice> stat;
   for (const auto &e : kernel_registry()) {
@@ -135,6 +137,9 @@ Choice choose(int kind, int64_t len, int prec, bool bwd, int need_tpb_div, bool 
     s.chain = e.chain;
     stat.push_back(s);
   }
+  if (few)
+    std::stable_sort(stat.begin(), stat.end(),
+                     [](const Choice &a, const Choice &b) { return a.e->tpt > b.e->tpt; });
   if (!stat.empty()) {
     const int pick = tune_pick(kind, len, prec, bwd, stat);
     if (pick >= 0) return stat[pick];

@@ -244,7 +244,13 @@ def test_convolutions(exe, tmp_path, dtype):
                         for n, hm, d, k in ((17, 300, -1, 0), (97, 17, 1, 1), (59, 33, -1, 0),
                                             (509, 3, 1, 0), (1009, 2, -1, 1), (1399, 2, 1, 0),
                                             (12289, 1, -1, 1), (10007, 2, 1, 0),
-                                            (20011, 1, -1, 0))])
+                                            (20011, 1, -1, 0))] + (
+        # Bluestein of few members (8 points a thread) and of many (16)
+        [P("c2c", n, hm, dtype, -1, node=f"bluestein_f64_fwd_n{M}_r{r}_t", cus=c)
+         for n, M, hm, c, r in ((58, 128, 9, 256, "8x2x8"), (58, 128, 40, 2, "16x8"),
+                                (458, 1024, 3, 256, "8x2x8x8"), (458, 1024, 9, 2, "16x4x16"),
+                                (838, 2048, 3, 256, "8x4x8x8"), (838, 2048, 5, 2, "16x8x16"))]
+        if dtype == "f64" else []))
 
 
 @pytest.mark.parametrize("dtype,direction,inplace", [("f32", -1, 0), ("f32", 1, 1), ("f64", -1, 0),
