@@ -45,8 +45,8 @@ void register_kernels_f32(std::vector<KEntry> &r) {
   PLF_DYNAMIC(k_c2c, KK_C2C, S, P,   64,   4, 16);
   PLF_DYNAMIC(k_c2c, KK_C2C, S, P,  256,   1, 16);
   // 15015 = 3.5.7.11.13 in one LDS pass on a compile-time chain: 4469 members
-  // 355 us (one block a CU, bound by its exchanges; 3.5.7.11.13 in five stages
-  // 390 to 411)
+  // 353 to 385 us by card (one block a CU, bound by its exchanges; 3.5.7.11.13
+  // in five stages 388 to 411)
   PLF_STATIC(k_c2c, KK_C2C, S, P, 1024,   1, 15, 13, 11, 7);
   PLF_DYNAMIC(k_c2c, KK_C2C, S, P, 1024,   1, 16);
 }
